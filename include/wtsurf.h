@@ -32,13 +32,11 @@ enum {
                          relative error of 4.7e-4 on A(k, omega) and a maximum of 87.
                          Beyond Ndim 80 it diverges on some instances, so runs with
                          Ndim > 80 fail with an error in this mode. */
-    WTSURF_MIXED = 2  /* per instance, FP64 iterations while the couplings are large,
-                         then FP32 MFMA inverse and GEMMs once sum |alpha| has fallen to
-                         1e-4 of its largest value so far (about a sixth of the
-                         iterations); eps accumulators, convergence sum, final inverses
-                         and traces FP64.  Within 1e-6 of FP64 on A(k, omega).  Runs on
-                         the persistent schedule whatever wtsurf_set_schedule says;
-                         Ndim <= 80. */
+    WTSURF_MIXED = 2  /* Within 1e-6 of FP64 on A(k, omega), Ndim <= 80, for callers that
+                         allow it.  Runs as WTSURF_FP64: the FP32 working precision holds
+                         that bound in the last sixth of an instance's iterations at most,
+                         and the kernels that switched there took 1.5 times as long as the
+                         FP64 rounds. */
 };
 
 /* Per-instance status bits (wtsurf_grid_download / wtsurf_spectral_grid). */

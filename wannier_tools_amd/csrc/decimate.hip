@@ -1,4 +1,6 @@
-// Batched Lopez-Sancho decimation on gfx950, FP64 and FP32-with-FP64-accumulation.
+// Batched Lopez-Sancho decimation on gfx950: the FP32-with-FP64-accumulation
+// rounds and the persistent schedules up to order 80, and the FP64 rounds
+// beyond (the FP64 rounds up to order 80 are in mid.hip).
 //
 // Restates surfgreen_1985 (src/surfgreen.f90:74-134) for many (k, omega)
 // instances.  Per iteration:
@@ -1515,8 +1517,8 @@ struct SlotWork {
     __device__ C *beta(int) const { return be; }
     __device__ C *alpha_next(int) const { return al; }
     __device__ C *beta_next(int) const { return be; }
-    __device__ SlotWork(void *work, int slot, size_t stride = bytes) {
-        unsigned char *base = reinterpret_cast<unsigned char *>(work) + (size_t)slot * stride;
+    __device__ SlotWork(void *work, int slot) {
+        unsigned char *base = reinterpret_cast<unsigned char *>(work) + (size_t)slot * bytes;
         C *c = reinterpret_cast<C *>(base);
         al = c;
         be = c + NN;
@@ -1890,106 +1892,6 @@ __global__ void __launch_bounds__(kBlock) persist_kernel(DecimateArgs a) {
     }
 }
 
-// Mixed precision (orders up to 80), persistent schedule.  Each instance runs
-// its iterations in FP64 while its couplings are large and switches to FP32
-// for the inverse and the GEMMs once sum |alpha| has fallen to kMixedSwitch of
-// its largest value so far.  The recursion squares the couplings, so from
-// there on each iteration's products are small against what eps_s and eps_t
-// have accumulated and their rounding no longer reaches A(k, omega) at the
-// 1e-6 level; the iterations before it (about five sixths of them) carry the
-// doubling amplification and stay FP64.  The eps accumulators, the
-// convergence sum, the three final inverses and the traces stay FP64 as in
-// the FP32 mode.  The slot is the FP64 one followed by alpha, beta, m1, m2 and
-// g in FP32 for the iterations after the switch.
-constexpr double kMixedSwitch = 1e-4;
-
-template <int Q>
-struct SlotWorkMixed {
-    static constexpr size_t NN = (size_t)(16 * Q) * (16 * Q);
-    static constexpr size_t bytes = SlotWork<Q, double>::bytes + 5 * NN * sizeof(float2);
-};
-
-// HALF: the order is at most 16 Q - 8 (dual_gemm_half).
-template <int Q, bool HALF>
-__global__ void __launch_bounds__(kBlock) persist_mixed_kernel(DecimateArgs a) {
-    extern __shared__ __align__(16) unsigned char lds[];
-    __shared__ Common<Q> cm;
-    __shared__ double red[kWaves];
-    constexpr int NN = 16 * Q * 16 * Q;
-    const int tid = threadIdx.x;
-    const int n = a.n;
-    const SlotWork<Q, double> w(a.work, blockIdx.x, SlotWorkMixed<Q>::bytes);
-    float2 *f = reinterpret_cast<float2 *>(reinterpret_cast<unsigned char *>(w.al) +
-                                           SlotWork<Q, double>::bytes);
-    float2 *al32 = f, *be32 = f + NN, *m1_32 = f + 2 * NN, *m2_32 = f + 3 * NN, *g32 = f + 4 * NN;
-    for (;;) {
-        if (setup_instance<Q, double, kBlock>(a, w, cm.s) == kDone) break;
-        int ik;
-        double2 z;
-        instance_of(a, uniform(cm.s.t), ik, z);
-        const double2 *H00 = a.hk + (size_t)ik * 2 * NN;
-        double peak = 0.0;
-        int low = 0;  // past the switch: FP32 inverse and GEMMs
-        for (;;) {
-            double asum;
-            if (!low) {
-                const bool sing = gj_inverse<Q, double, kBlock>(lds, lds + GjLay<Q, double>::S, cm,
-                                                                w.es, w.et, H00, z, n, 4, nullptr,
-                                                                w.g);
-                if (tid == 0 && sing) cm.s.status |= 1;
-                dual_gemm_any<Q, double, 0, HALF>(lds, red, w.al, w.be, w.g, n, w.m1, w.m2, nullptr);
-                __syncthreads();
-                dual_gemm_any<Q, double, 1, HALF>(lds, red, w.m1, w.m2, w.be, n, nullptr, w.be, w.es);
-                __syncthreads();
-                asum = dual_gemm_any<Q, double, 2, HALF>(lds, red, w.m2, w.m1, w.al, n, nullptr, w.al, w.et);
-            } else {
-                const bool sing = gj_inverse<Q, float, kBlock>(lds, lds + GjLay<Q, float>::S, cm,
-                                                               w.es, w.et, H00, z, n, 4, nullptr,
-                                                               g32);
-                if (tid == 0 && sing) cm.s.status |= 1;
-                dual_gemm_any<Q, float, 0, HALF>(lds, red, al32, be32, g32, n, m1_32, m2_32, nullptr);
-                __syncthreads();
-                dual_gemm_any<Q, float, 1, HALF>(lds, red, m1_32, m2_32, be32, n, nullptr, be32, w.es);
-                __syncthreads();
-                asum = dual_gemm_any<Q, float, 2, HALF>(lds, red, m2_32, m1_32, al32, n, nullptr, al32, w.et);
-            }
-            const int it = uniform(cm.s.it);
-            const int converged = uniform(asum <= a.accuracy ? 1 : 0);
-            peak = fmax(peak, asum);
-            const int go_low = uniform(!low && asum <= kMixedSwitch * peak ? 1 : 0);
-            __syncthreads();
-            if (converged) break;
-            if (it >= a.itermax) {
-                if (tid == 0) cm.s.status |= 2;
-                break;
-            }
-            if (go_low) {  // alpha and beta to FP32 for the rest of the instance
-                for (int e = tid; e < NN; e += kBlock) {
-                    const double2 x = w.al[e], y = w.be[e];
-                    al32[e] = make_float2((float)x.x, (float)x.y);
-                    be32[e] = make_float2((float)y.x, (float)y.y);
-                }
-                low = 1;
-                __syncthreads();
-            }
-            if (tid == 0) cm.s.it = it + 1;
-        }
-        for (int q = 0; q < 3; ++q) {
-            double2 *full = a.gfull ? a.gfull + ((size_t)cm.s.t * 3 + q) * n * n : nullptr;
-            const double2 *eps = q == 1 ? w.et : w.es;
-            const double2 *eps2 = q == 2 ? w.et : nullptr;
-            const bool sing = gj_inverse<Q, double, kBlock>(lds, lds + GjLay<Q, double>::S, cm,
-                                                            eps, eps2, H00, z, n, full ? 2 : 1,
-                                                            full, nullptr);
-            if (tid == 0) {
-                if (sing) cm.s.status |= 1;
-                final_traces<Q>(a, cm, LdsInverse<Q>{lds, cm}, q, ik);
-            }
-            __syncthreads();
-        }
-    }
-}
-
 constexpr int kMaxQ = 24;
 constexpr int kRoundsPerBatch = 8;
 
@@ -2003,8 +1905,10 @@ int decimate_max_q() { return kMaxQ; }
 
 template <int Q, typename R>
 static int launch_round(const DecimateArgs &a, int per_set, int set, bool gj, hipStream_t s) {
-    if constexpr (Q > 5 && std::is_same_v<R, float>) {
-        return -1;  // no FP32 kernels beyond order 80 (the C ABI refuses that case)
+    if constexpr ((Q > 5) == std::is_same_v<R, float>) {
+        // no FP32 kernels beyond order 80 (the C ABI refuses that case); FP64
+        // rounds up to order 80 are mid.hip's
+        return -1;
     } else if constexpr (Q <= 5) {
         constexpr size_t gj_lds = GjLay<Q, R>::bytes;
         if (gj)
@@ -2060,10 +1964,10 @@ static size_t dispatch_slot_bytes(int q) {
 template <int Q, typename R>
 static void allow_lds() {
     hipError_t e;
-    if constexpr (Q <= 5)
+    if constexpr (Q <= 5 && std::is_same_v<R, float>)
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gj_round_kernel<Q, R>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)GjLay<Q, R>::bytes);
-    else if constexpr (std::is_same_v<R, double>)
+    else if constexpr (Q > 5 && std::is_same_v<R, double>)
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gj_large_round_kernel<Q, R>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)GjLayL<Q>::bytes);
     else
@@ -2087,19 +1991,7 @@ int decimate_slots_per_set(int ninst, int num_cu) {
     return half < num_cu ? (half > 0 ? half : 1) : num_cu;
 }
 
-static size_t mixed_slot_bytes(int q) {
-    switch (q) {
-        case 1: return SlotWorkMixed<1>::bytes;
-        case 2: return SlotWorkMixed<2>::bytes;
-        case 3: return SlotWorkMixed<3>::bytes;
-        case 4: return SlotWorkMixed<4>::bytes;
-        case 5: return SlotWorkMixed<5>::bytes;
-        default: return 0;
-    }
-}
-
 size_t decimate_slot_bytes(int q, int precision) {
-    if (precision == 2) return mixed_slot_bytes(q);
     return precision == 0 ? dispatch_slot_bytes<double>(q) : dispatch_slot_bytes<float>(q);
 }
 
@@ -2189,33 +2081,6 @@ static int launch_persist(const DecimateArgs &a, int nblocks, hipStream_t s) {
     }
 }
 
-template <int Q>
-static int launch_persist_mixed(const DecimateArgs &a, int nblocks, hipStream_t s) {
-    constexpr size_t lds = PersistLay<Q, double>::bytes;
-    auto go = [&](auto kernel) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-            (void)hipGetLastError();
-        hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(kBlock), lds, s, a);
-    };
-    if (Q >= 2 && a.n <= 16 * Q - 8)
-        go(persist_mixed_kernel<Q, (Q >= 2)>);
-    else
-        go(persist_mixed_kernel<Q, false>);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
-static int dispatch_persist_mixed(const DecimateArgs &a, int q, int nblocks, hipStream_t s) {
-    switch (q) {
-        case 1: return launch_persist_mixed<1>(a, nblocks, s);
-        case 2: return launch_persist_mixed<2>(a, nblocks, s);
-        case 3: return launch_persist_mixed<3>(a, nblocks, s);
-        case 4: return launch_persist_mixed<4>(a, nblocks, s);
-        case 5: return launch_persist_mixed<5>(a, nblocks, s);
-        default: return -1;
-    }
-}
-
 template <typename R>
 static int dispatch_persist(const DecimateArgs &a, int q, int nblocks, hipStream_t s) {
     switch (q) {
@@ -2234,7 +2099,6 @@ int decimate_persistent_run(const DecimateArgs &a, int q, int precision, int nbl
                             hipStream_t s) {
     if (q < 1 || q > decimate_persistent_max_q() || nblocks < 1) return -1;
     if (hipMemsetAsync(a.queue, 0, 2 * sizeof(unsigned), s) != hipSuccess) return -1;
-    if (precision == 2) return dispatch_persist_mixed(a, q, nblocks, s);
     return precision == 0 ? dispatch_persist<double>(a, q, nblocks, s)
                           : dispatch_persist<float>(a, q, nblocks, s);
 }

@@ -55,8 +55,8 @@ struct DevBuf {
 // first call on a device, with that device current.  Layout (256-byte aligned
 // pieces):
 //   hk    padded H00, H01              2 NP^2 complex double
-//   work  two decimation slots         2 slot_bytes_lds_fp64(Q)
-//   state two SlotState, queue [2]
+//   work  two decimation slots         2 slot_bytes_lds_fp64(Q), or one of mid.hip
+//   state two SlotState or MidState, queue [2]
 //   gfull GLL, GRR, GB                 3 n^2 complex double
 //   outs  dos_l, dos_r, dos_bulk; iters, status, an empty orbital list
 namespace {
@@ -66,8 +66,10 @@ constexpr size_t kAlign = 256;
 constexpr size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
 constexpr size_t kOffHk = 0;
 constexpr size_t kOffWork = kOffHk + align_up((size_t)2 * kNoallocNP * kNoallocNP * sizeof(double2));
-constexpr size_t kOffState = kOffWork + align_up((size_t)kSlotSets * slot_bytes_lds_fp64(kNoallocNP / 16));
-constexpr size_t kOffQueue = kOffState + align_up((size_t)kSlotSets * sizeof(SlotState));
+constexpr size_t kOffState =
+    kOffWork + align_up(std::max((size_t)kSlotSets * slot_bytes_lds_fp64(kNoallocNP / 16), kMidMaxSlotBytes));
+constexpr size_t kOffQueue =
+    kOffState + align_up((size_t)kSlotSets * std::max(sizeof(SlotState), sizeof(MidState)));
 constexpr size_t kOffG = kOffQueue + kAlign;
 constexpr size_t kOffOut = kOffG + align_up((size_t)3 * kNoallocMaxN * kNoallocMaxN * sizeof(double2));
 constexpr size_t kNoallocScratchBytes = kOffOut + kAlign;
@@ -153,6 +155,7 @@ struct wtsurf_ctx {
     DevBuf<unsigned char> work, state;
     DevBuf<unsigned> queue;
     int per_set = 0;
+    MidPlan plan;        // slots of the last ensure_work for mid.hip's rounds
     bool ran = false;    // a grid run is queued or done (wtsurf_grid_download)
     bool timed = false;  // ev[0..2] bracket the last grid or batch run
 
@@ -202,7 +205,26 @@ static int sync_orbitals(wtsurf_ctx *c) {
     return 0;
 }
 
-static int ensure_work(wtsurf_ctx *c, int q, int precision, int ninst) {
+// FP64 rounds of orders up to 80 (mid.hip): the schedule asked for is the
+// rounds, or automatic above the small kernel's orders.
+static bool use_mid(const wtsurf_ctx *c, int n, int precision) {
+    if (precision != WTSURF_FP64 || n > decimate_mid_max_n()) return false;
+    if (c->schedule == WTSURF_SCHEDULE_PERSISTENT) return false;
+    return c->schedule == WTSURF_SCHEDULE_ROUNDS || n > decimate_small_max_n();
+}
+
+static int ensure_work(wtsurf_ctx *c, int n, int precision, int ninst) {
+    if (use_mid(c, n, precision)) {
+        c->plan = decimate_mid_plan(ninst, c->num_cu);
+        const size_t slots = (size_t)c->plan.sets * c->plan.per_set;
+        const size_t want = slots * decimate_mid_slot_bytes(n);
+        if (want > c->work.n && (c->work.release(), c->work.ensure(want)))
+            return c->fail("out of device memory (decimation workspace)");
+        if (c->state.ensure(2 * slots * sizeof(MidState)) || c->queue.ensure(2))
+            return c->fail("out of device memory (slot state)");
+        return 0;
+    }
+    const int q = padded_q(n);
     const size_t per_slot = decimate_slot_bytes(q, precision);
     if (per_slot == 0) return c->fail("no decimation kernel for this order");
     const int per_set = decimate_slots_per_set(ninst, c->num_cu);
@@ -426,9 +448,10 @@ struct RunBufs {
     double *dos_l = nullptr, *dos_r = nullptr, *dos_b = nullptr;
     int *iters = nullptr, *status = nullptr;
     void *work = nullptr;
-    SlotState *state = nullptr;
+    void *state = nullptr;  // SlotState or MidState records
     unsigned *queue = nullptr;
     int per_set = 0;
+    MidPlan plan;
 };
 
 // Enqueue the rounds of one decimation run on the context streams.
@@ -442,7 +465,7 @@ static int run_decimation(wtsurf_ctx *c, const RunBufs &b, int ninst, int nk, in
     a.eta0 = eta; a.nk = nk; a.nomega = nomega; a.ninst = ninst; a.n = n; a.nw = nw;
     a.itermax = c->itermax; a.accuracy = c->accuracy;
     a.top = d_top; a.ntop = ntop; a.bot = d_bot; a.nbot = nbot; a.divisor = divisor;
-    a.work = b.work; a.state = b.state; a.queue = b.queue;
+    a.work = b.work; a.state = static_cast<SlotState *>(b.state); a.queue = b.queue;
     a.dos_l = b.dos_l; a.dos_r = b.dos_r; a.dos_bulk = b.dos_b;
     a.iters = b.iters; a.status = b.status; a.gfull = gfull;
     if (spin) {
@@ -459,10 +482,7 @@ static int run_decimation(wtsurf_ctx *c, const RunBufs &b, int ninst, int nk, in
         }
         return 0;
     }
-    // the mixed precision switches per instance, which only the persistent
-    // schedule (whole instances per workgroup) can follow
-    if ((c->schedule == WTSURF_SCHEDULE_PERSISTENT || precision == WTSURF_MIXED) &&
-        q <= decimate_persistent_max_q()) {
+    if (c->schedule == WTSURF_SCHEDULE_PERSISTENT && q <= decimate_persistent_max_q()) {
         // one workgroup per CU (at most one per instance), slots 0.. of the workspace
         const int nblocks = std::min(c->num_cu, ninst);
         if (nblocks > kSlotSets * b.per_set) return c->fail("decimation workspace too small");
@@ -479,7 +499,9 @@ static int run_decimation(wtsurf_ctx *c, const RunBufs &b, int ninst, int nk, in
     ctl.s[kSlotSets] = c->cnt;
     for (int i = 0; i < kRoundEvents; ++i) ctl.ev[i] = c->drv[i];
     ctl.pinned = c->pinned;
-    if (int r = decimate_run(a, q, precision, b.per_set, ctl)) {
+    const bool mid = use_mid(c, n, precision);
+    if (int r = mid ? decimate_mid_run(a, b.plan, static_cast<MidState *>(b.state), c->num_cu, ctl)
+                    : decimate_run(a, q, precision, b.per_set, ctl)) {
         for (auto s : c->aux) (void)hipStreamSynchronize(s);  // rounds already queued there
         (void)hipStreamSynchronize(c->cnt);
         if (r == -2) return c->fail("decimation made no progress within its round bound");
@@ -510,7 +532,10 @@ static int launch_decimation(wtsurf_ctx *c, int ninst, int nk, int nomega, const
                              const int *d_bot, int nbot, int precision,
                              InstanceLists inst = InstanceLists()) {
     if (int r = check_order(c, n, precision)) return r;
-    if (int r = ensure_work(c, padded_q(n), precision, ninst)) return r;
+    // The mixed precision was FP64 but for the last sixth of the iterations;
+    // the FP64 rounds now take two thirds of the time those took.
+    if (precision == WTSURF_MIXED) precision = WTSURF_FP64;
+    if (int r = ensure_work(c, n, precision, ninst)) return r;
     if (c->dos_l.ensure(ninst) || c->dos_r.ensure(ninst) || c->dos_b.ensure(ninst) ||
         c->iters.ensure(ninst) || c->status.ensure(ninst))
         return c->fail("out of device memory (outputs)");
@@ -518,8 +543,9 @@ static int launch_decimation(wtsurf_ctx *c, int ninst, int nk, int nomega, const
     b.hk = c->hk.p;
     b.dos_l = c->dos_l.p; b.dos_r = c->dos_r.p; b.dos_b = c->dos_b.p;
     b.iters = c->iters.p; b.status = c->status.p;
-    b.work = c->work.p; b.state = reinterpret_cast<SlotState *>(c->state.p); b.queue = c->queue.p;
+    b.work = c->work.p; b.state = c->state.p; b.queue = c->queue.p;
     b.per_set = c->per_set;
+    b.plan = c->plan;
     c->spin_ninst = 0;
     double *spin = nullptr;
     if (c->spin_mode != WTSURF_SPIN_OFF) {
@@ -558,7 +584,7 @@ int wtsurf_surfgreen_1985(wtsurf_ctx *c, int n, double omega, double eta, const 
     // buffers of their own (grown on demand, kept for the next call), so that
     // the grid's H00/H01, energies and outputs stay as the last grid run left them
     if (c->hk1.ensure(pad.size()) || c->one_d.ensure(4) || c->one_i.ensure(3) ||
-        c->gfull.ensure((size_t)3 * n * n) || ensure_work(c, padded_q(n), WTSURF_FP64, 1))
+        c->gfull.ensure((size_t)3 * n * n) || ensure_work(c, n, WTSURF_FP64, 1))
         return c->fail("out of device memory");
     WT_HIP(c, hipMemcpy(c->hk1.p, pad.data(), pad.size() * sizeof(double2), hipMemcpyHostToDevice));
     WT_HIP(c, hipMemcpy(c->one_d.p + 3, &omega, sizeof(double), hipMemcpyHostToDevice));
@@ -566,8 +592,9 @@ int wtsurf_surfgreen_1985(wtsurf_ctx *c, int n, double omega, double eta, const 
     b.hk = c->hk1.p;
     b.dos_l = c->one_d.p; b.dos_r = c->one_d.p + 1; b.dos_b = c->one_d.p + 2;
     b.iters = c->one_i.p; b.status = c->one_i.p + 1;
-    b.work = c->work.p; b.state = reinterpret_cast<SlotState *>(c->state.p); b.queue = c->queue.p;
+    b.work = c->work.p; b.state = c->state.p; b.queue = c->queue.p;
     b.per_set = c->per_set;
+    b.plan = c->plan;
     // traces are not needed here: empty orbital lists (pointing at a valid int)
     if (int r = run_decimation(c, b, 1, 1, 1, c->one_d.p + 3, eta, 1.0, c->gfull.p, n, n,
                                c->one_i.p + 2, 0, c->one_i.p + 2, 0, WTSURF_FP64, InstanceLists(),
@@ -617,7 +644,7 @@ int wtsurf_surfgreen_1985_noalloc(wtsurf_ctx *c, int n, double omega, double eta
     b.dos_l = outs; b.dos_r = outs + 1; b.dos_b = outs + 2;
     b.iters = iouts; b.status = iouts + 1;
     b.work = base + kOffWork;
-    b.state = reinterpret_cast<SlotState *>(base + kOffState);
+    b.state = base + kOffState;
     b.queue = reinterpret_cast<unsigned *>(base + kOffQueue);
     b.per_set = 1;
     if (int r = run_decimation(c, b, 1, 1, 1, nullptr, eta, 1.0, gfull, n, n, iouts + 2, 0,

@@ -75,8 +75,7 @@ constexpr size_t slot_bytes_lds_fp64(int q) { return (size_t)7 * (16 * q) * (16 
 int decimate_max_q();       // largest Q the decimation kernels are built for
 // Slots per stream set for ninst instances on num_cu CUs (one of each kernel per CU).
 int decimate_slots_per_set(int ninst, int num_cu);
-// precision: 0 = FP64, 1 = FP32 inverse/GEMMs with FP64 accumulation and finals,
-// 2 = mixed (FP64 iterations, then FP32 ones past the switch; persistent only)
+// precision: 0 = FP64, 1 = FP32 inverse/GEMMs with FP64 accumulation and finals
 size_t decimate_slot_bytes(int q, int precision);
 // Enqueues the decimation of a.ninst instances on the work streams
 // ctl.s[0..kSlotSets) and returns once every instance is counted finished
@@ -96,6 +95,29 @@ int decimate_persistent_run(const DecimateArgs &a, int q, int precision, int nbl
 // a.state unused).  Returns once the launch is queued on s.
 int decimate_small_max_n();
 int decimate_small_run(const DecimateArgs &a, int num_cu, hipStream_t s);
+
+// FP64 orders up to decimate_mid_max_n() as rounds of two kernels with the
+// inverse in registers (mid.hip).  State of one slot between rounds; two per
+// slot (a round reads one and writes the other).
+struct MidState {
+    int phase;   // empty, in an iteration, done
+    int t;       // instance id
+    int it;      // current iteration (1-based)
+    int status;  // bit0 singular solve, bit1 not converged
+    int buf;     // which of the slot's two states the iteration reads
+    int pad;
+};
+struct MidPlan {
+    int sets = 1, per_set = 1;  // slot sets (one stream each) and slots per set
+};
+constexpr size_t kMidMaxSlotBytes = (size_t)922112;  // slot of order 80
+int decimate_mid_max_n();
+size_t decimate_mid_slot_bytes(int n);
+MidPlan decimate_mid_plan(int ninst, int num_cu);
+// a.work: sets * per_set slots of decimate_mid_slot_bytes(a.n); state: 2 * sets
+// * per_set records.  As decimate_run otherwise (-2: no progress).
+int decimate_mid_run(const DecimateArgs &a, const MidPlan &plan, MidState *state, int num_cu,
+                     const RoundCtl &ctl);
 
 // Fourier sum H00(k), H01(k) (src/ham_qlayer2qlayer.f90:45-97).
 struct FourierArgs {
