@@ -13,12 +13,18 @@
 //
 //   C(p1, p2) = sum_{c1 < m1, c2 < m2} sum_f E_f(c1, c2) a_f((c1 + p1) mod m1, (c2 + p2) mod m2)
 //
-// with out(iq1, iq2) = C((iq1 - 1) mod m1, (iq2 - 1) mod m2).  The correlation
-// kernel takes one p2 per workgroup and one p1 per thread: per c2 it stages
-// the row E_f(:, c2) and the row a_f(:, (c2 + p2) mod m2) twice over (so that
-// c1 + p1 needs no wrap) in LDS; every thread then reads the E row at one
-// address (broadcast) and the a row at consecutive addresses.  The sum is
-// O((m1 m2)^2) FP64 multiply-adds, milliseconds at a 257 x 257 plane.
+// with out(iq1, iq2) = C((iq1 - 1) mod m1, (iq2 - 1) mod m2): O((m1 m2)^2) FP64
+// multiply-adds, summed as they stand (a transform would leave an absolute
+// error of the largest C everywhere, and the fields' peaks span decades).
+// correlate_kernel takes R2 values of p2 and all p1 per workgroup, 8
+// consecutive p1 per thread: a thread slides an 8-wide window of each of its
+// R2 rows of a_f over the row of E_f, one LDS read of a row and one of E
+// (broadcast) for 8 R2 multiply-adds, where a thread per (p1, p2) took two
+// reads for each: at 257 x 257, moduli 256 and four fields, 6.97 ms, bound by
+// the LDS reads, and 0.79 ms now.  Rows go in groups of G values of c2, one per group of
+// threads; the sum over c2 is cut into slices so that there are workgroups for
+// the whole chip, and expand_kernel adds the slices in order.  Bound by the
+// FP64 vector ALUs.
 //
 // 2. Linear autocorrelation along a k path, per energy (surfstat_jdos,
 // src/surfstat.f90:891-907): with h = (nk - 1)/2 and s = iq - h,
@@ -55,56 +61,116 @@ __global__ void __launch_bounds__(kCorrBlock) fold_kernel(const double *__restri
     }
 }
 
-// C(p1, p2): block (p2, p1 tile); dynamic LDS 3 m1 doubles.
-__global__ void __launch_bounds__(kCorrBlock) correlate_kernel(const double *__restrict__ a,
-                                                               const double *__restrict__ e,
-                                                               int nkx, int nky, int m1, int m2,
-                                                               int nfield, double *__restrict__ c) {
+// Place of element x of a row of a in LDS: one double of padding in eight, so
+// that the threads' windows (8 apart) fall on different banks.
+__device__ __forceinline__ int skew(int x) { return x + (x >> 3); }
+
+// Slice blockIdx.y of C(p1, p2) for p2 = R2 blockIdx.x ..: threads tp = tid % TP
+// (p1 = 8 tp .. 8 tp + 7) of group g = tid / TP (c2 = c20 + g of each chunk).
+// part [slices][m2][m1].  Dynamic LDS: G rows of E, G + R2 - 1 skewed rows of a.
+template <int R2>
+__global__ void __launch_bounds__(kCorrBlock) correlate_kernel(
+    const double *__restrict__ a, const double *__restrict__ e, int nkx, int nky, int m1, int m2,
+    int nfield, int TP, int len, double *__restrict__ part) {
     extern __shared__ __align__(16) double lds[];
-    double *erow = lds;        // [m1]
-    double *arow = lds + m1;   // [2 m1]: a_f(j mod m1, r)
-    const int p2 = blockIdx.x;
-    const int p1 = blockIdx.y * kCorrBlock + threadIdx.x;
-    double acc = 0.0;
-    for (int c2 = 0; c2 < m2; ++c2) {
-        int r = c2 + p2;
-        if (r >= m2) r -= m2;
-        for (int f = 0; f < nfield; ++f) {
-            const double *ef = e + ((size_t)f * m2 + c2) * m1;
-            const double *af = a + (size_t)f * nkx * nky + (size_t)nkx * r;
-            __syncthreads();  // the previous rows are no longer read
-            for (int j = threadIdx.x; j < m1; j += kCorrBlock) {
-                erow[j] = ef[j];
-                const double v = af[j];
-                arow[j] = v;
-                arow[j + m1] = v;
-            }
-            __syncthreads();
-            if (p1 < m1) {
-                const double *ar = arow + p1;
-                double s0 = 0.0, s1 = 0.0;
-                int c1 = 0;
-                for (; c1 + 1 < m1; c1 += 2) {
-                    s0 = fma(erow[c1], ar[c1], s0);
-                    s1 = fma(erow[c1 + 1], ar[c1 + 1], s1);
+    const int G = kCorrBlock / TP;
+    const int ld = skew(len) + 1;
+    double *er = lds;               // [G][m1]
+    double *ar = lds + (size_t)G * m1;  // [G + R2 - 1][ld]
+    const int tid = threadIdx.x;
+    const int tp = tid % TP, g = tid / TP;
+    const int p20 = R2 * blockIdx.x;
+    const int chunks = (m2 + G - 1) / G;  // per field
+    const long total = (long)nfield * chunks;
+    const long k0 = total * blockIdx.y / gridDim.y, k1 = total * (blockIdx.y + 1) / gridDim.y;
+    double acc[R2][8];
+#pragma unroll
+    for (int j = 0; j < R2; ++j)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[j][i] = 0.0;
+    for (long k = k0; k < k1; ++k) {
+        const int f = (int)(k / chunks), c20 = (int)(k - (long)f * chunks) * G;
+        const int ng = min(G, m2 - c20);  // rows of this chunk
+        const double *ef = e + ((size_t)f * m2 + c20) * m1;
+        const double *af = a + (size_t)f * nkx * nky;
+        __syncthreads();  // the previous rows are no longer read
+        for (int j = tid; j < ng * m1; j += kCorrBlock) er[j] = ef[j];
+        for (int row = 0; row < ng + R2 - 1; ++row) {
+            const double *src = af + (size_t)nkx * ((c20 + p20 + row) % m2);
+            for (int j = tid; j < len; j += kCorrBlock) ar[row * ld + skew(j)] = src[j % m1];
+        }
+        __syncthreads();
+        if (g < ng) {
+            const double *eg = er + g * m1;
+            const double *w0 = ar + g * ld + 9 * tp;  // window of p2 = p20 + j: row g + j
+            double w[R2][8];
+#pragma unroll
+            for (int j = 0; j < R2; ++j)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) w[j][i] = w0[j * ld + i];
+            int c1 = 0;
+            for (; c1 + 8 <= m1; c1 += 8) {
+                w0 += 9;
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const double ev = eg[c1 + t];
+#pragma unroll
+                    for (int j = 0; j < R2; ++j) {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) acc[j][i] = fma(ev, w[j][(t + i) & 7], acc[j][i]);
+                        w[j][t] = w0[j * ld + t];
+                    }
                 }
-                if (c1 < m1) s0 = fma(erow[c1], ar[c1], s0);
-                acc += s0 + s1;
             }
+            w0 += 9;
+#pragma unroll
+            for (int t = 0; t < 7; ++t)
+                if (c1 + t < m1) {
+                    const double ev = eg[c1 + t];
+#pragma unroll
+                    for (int j = 0; j < R2; ++j) {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) acc[j][i] = fma(ev, w[j][(t + i) & 7], acc[j][i]);
+                        w[j][t] = w0[j * ld + t];
+                    }
+                }
         }
     }
-    if (p1 < m1) c[(size_t)p2 * m1 + p1] = acc;
+    // the groups' sums, added in order
+    __syncthreads();
+    for (int j = 0; j < R2; ++j) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            double v = acc[0][i];
+#pragma unroll
+            for (int q = 1; q < R2; ++q)
+                if (j == q) v = acc[q][i];
+            lds[(g * 8 + i) * TP + tp] = v;
+        }
+        __syncthreads();
+        if (p20 + j < m2)
+            for (int p1 = tid; p1 < m1; p1 += kCorrBlock) {
+                double v = 0.0;
+                for (int q = 0; q < G; ++q) v += lds[(q * 8 + (p1 & 7)) * TP + (p1 >> 3)];
+                part[((size_t)blockIdx.y * m2 + p20 + j) * m1 + p1] = v;
+            }
+        __syncthreads();
+    }
 }
 
-// out(iq1, iq2) = C((iq1 - 1) mod m1, (iq2 - 1) mod m2); out [nky][nkx].
+// out(iq1, iq2) = C((iq1 - 1) mod m1, (iq2 - 1) mod m2), C the sum of its slices;
+// out [nky][nkx].
 __global__ void __launch_bounds__(kCorrBlock) expand_kernel(const double *__restrict__ c, int nkx,
-                                                            int nky, int m1, int m2,
+                                                            int nky, int m1, int m2, int slices,
                                                             double *__restrict__ out) {
     const long total = (long)nkx * nky;
     for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < total;
          t += (long)gridDim.x * blockDim.x) {
         const int i1 = (int)(t % nkx), i2 = (int)(t / nkx);
-        out[t] = c[(size_t)(i2 % m2) * m1 + (i1 % m1)];
+        const double *p = c + (size_t)(i2 % m2) * m1 + (i1 % m1);
+        double s = 0.0;
+        for (int q = 0; q < slices; ++q) s += p[(size_t)q * m1 * m2];
+        out[t] = s;
     }
 }
 
@@ -141,6 +207,35 @@ int kpath_jdos_launch(const double *fields, int nk, int nomega, int nfield, doub
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
+// Launch shape of correlate_kernel: threads along p1 (a power of two, so that
+// the groups of threads tile the workgroup), the LDS length of a row of a, R2
+// as large as two workgroups of LDS a CU allow, and slices for about four
+// workgroups a CU.
+struct CorrPlan {
+    int tp, len, r2, slices;
+    size_t lds;
+};
+static CorrPlan corr_plan(int m1, int m2, int nfield) {
+    CorrPlan p{};
+    p.tp = 8;
+    while (8 * p.tp < m1) p.tp *= 2;
+    p.len = m1 + 8 * p.tp + 8;
+    const int G = kCorrBlock / p.tp;
+    for (p.r2 = 4;; p.r2 /= 2) {
+        const size_t rows = (size_t)G * m1 + (size_t)(G + p.r2 - 1) * (p.len + p.len / 8 + 1);
+        p.lds = std::max(rows, (size_t)8 * kCorrBlock) * sizeof(double);
+        if (p.r2 == 1 || p.lds <= (size_t)80 * 1024) break;
+    }
+    const long blocks = (m2 + p.r2 - 1) / p.r2;
+    const long chunks = (long)nfield * ((m2 + G - 1) / G);
+    p.slices = (int)std::max<long>(1, std::min(chunks, (1024 + blocks - 1) / blocks));
+    return p;
+}
+
+size_t kplane_corr_doubles(int m1, int m2, int nfield) {
+    return (size_t)corr_plan(m1, m2, nfield).slices * m1 * m2;
+}
+
 int kplane_corr_launch(const KplaneCorrArgs &k, hipStream_t s) {
     if (k.nkx < 1 || k.nky < 1 || k.m1 < 1 || k.m2 < 1 || k.m1 > k.nkx || k.m2 > k.nky ||
         k.m1 > kKplaneMaxM || k.nfield < 1)
@@ -149,14 +244,26 @@ int kplane_corr_launch(const KplaneCorrArgs &k, hipStream_t s) {
     const int gfold = (int)std::min<long>((nfold + kCorrBlock - 1) / kCorrBlock, 4096);
     hipLaunchKernelGGL(fold_kernel, dim3(gfold), dim3(kCorrBlock), 0, s, k.fields, k.nkx, k.nky,
                        k.m1, k.m2, k.nfield, k.folded);
-    const dim3 grid(k.m2, (k.m1 + kCorrBlock - 1) / kCorrBlock);
-    const size_t lds = (size_t)3 * k.m1 * sizeof(double);
-    hipLaunchKernelGGL(correlate_kernel, grid, dim3(kCorrBlock), lds, s, k.fields, k.folded, k.nkx,
-                       k.nky, k.m1, k.m2, k.nfield, k.corr);
+    const CorrPlan p = corr_plan(k.m1, k.m2, k.nfield);
+    auto go = [&](auto kernel) {
+        if (p.lds > (size_t)64 * 1024 &&
+            hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds) != hipSuccess)
+            (void)hipGetLastError();  // the launch reports whether the size is accepted
+        hipLaunchKernelGGL(kernel, dim3((k.m2 + p.r2 - 1) / p.r2, p.slices), dim3(kCorrBlock), p.lds,
+                           s, k.fields, k.folded, k.nkx, k.nky, k.m1, k.m2, k.nfield, p.tp, p.len,
+                           k.corr);
+    };
+    if (p.r2 == 4)
+        go(correlate_kernel<4>);
+    else if (p.r2 == 2)
+        go(correlate_kernel<2>);
+    else
+        go(correlate_kernel<1>);
     const long nout = (long)k.nkx * k.nky;
     const int gout = (int)std::min<long>((nout + kCorrBlock - 1) / kCorrBlock, 4096);
     hipLaunchKernelGGL(expand_kernel, dim3(gout), dim3(kCorrBlock), 0, s, k.corr, k.nkx, k.nky,
-                       k.m1, k.m2, k.out);
+                       k.m1, k.m2, p.slices, k.out);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

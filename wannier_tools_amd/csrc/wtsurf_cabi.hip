@@ -137,6 +137,7 @@ struct wtsurf_ctx {
     int nk = 0, nomega = 0;
     DevBuf<double> kpts, omega;
     DevBuf<double2> phase, hk;
+    DevBuf<double> qpi;  // fields, scratch and result of the QPI sums
     DevBuf<double> dos_l, dos_r, dos_b;
     DevBuf<int> iters, status;
     // per-instance batch (wtsurf_spectral_batch)
@@ -281,6 +282,7 @@ void wtsurf_ctx_destroy(wtsurf_ctx *c) {
     c->hr.release(); c->irvec.release(); c->slot_begin.release();
     c->d_top.release(); c->d_bot.release();
     c->kpts.release(); c->omega.release(); c->phase.release(); c->hk.release();
+    c->qpi.release();
     c->dos_l.release(); c->dos_r.release(); c->dos_b.release();
     c->inst_k.release(); c->inst_w.release(); c->inst_eta.release(); c->spin.release();
     c->iters.release(); c->status.release(); c->work.release(); c->state.release();
@@ -807,15 +809,16 @@ int wtsurf_kplane_autocorrelation(wtsurf_ctx *c, int nkx, int nky, int m1, int m
     if (m1 > kplane_corr_max_m()) return c->fail("k-plane too large for the autocorrelation kernel");
     if (int r = use_device(c)) return r;
     const size_t plane = (size_t)nkx * nky;
-    DevBuf<double> buf;
-    if (buf.ensure((size_t)nfield * plane + (size_t)(nfield + 1) * m1 * m2 + plane))
+    DevBuf<double> &buf = c->qpi;  // grown on demand, kept for the next call
+    const size_t corr = kplane_corr_doubles(m1, m2, nfield);
+    if (buf.ensure((size_t)nfield * plane + (size_t)nfield * m1 * m2 + corr + plane))
         return c->fail("out of device memory (k-plane autocorrelation)");
     KplaneCorrArgs k{};
     k.fields = buf.p;
     k.nkx = nkx; k.nky = nky; k.m1 = m1; k.m2 = m2; k.nfield = nfield;
     k.folded = buf.p + (size_t)nfield * plane;
     k.corr = k.folded + (size_t)nfield * m1 * m2;
-    k.out = k.corr + (size_t)m1 * m2;
+    k.out = k.corr + corr;
     int rc = 0;
     hipError_t e;
     if ((e = hipMemcpyAsync(buf.p, fields, (size_t)nfield * plane * sizeof(double),
@@ -828,7 +831,6 @@ int wtsurf_kplane_autocorrelation(wtsurf_ctx *c, int nkx, int nky, int m1, int m
              (e = hipStreamSynchronize(c->stream)) != hipSuccess)
         rc = c->hipfail(e, "download");
     if (rc) (void)hipStreamSynchronize(c->stream);
-    buf.release();
     return rc;
 }
 

@@ -136,15 +136,16 @@ struct FourierArgs {
 int fourier_launch(const FourierArgs &a, hipStream_t s);
 
 // QPI autocorrelation over a k-plane (src/fermiarc.f90:496-560), device buffers.
-constexpr int kKplaneMaxM = 2048;  // largest m1 (LDS rows of 3 m1 doubles)
+constexpr int kKplaneMaxM = 2048;  // largest m1 (rows in LDS)
 struct KplaneCorrArgs {
     const double *fields;   // [nfield][nky][nkx]
     int nkx, nky, m1, m2, nfield;
     double *folded;         // [nfield][m2][m1] scratch
-    double *corr;           // [m2][m1] scratch
+    double *corr;           // kplane_corr_doubles() scratch: [slices][m2][m1]
     double *out;            // [nky][nkx]
 };
 int kplane_corr_max_m();
+size_t kplane_corr_doubles(int m1, int m2, int nfield);
 int kplane_corr_launch(const KplaneCorrArgs &k, hipStream_t s);
 // k-path joint density of states (src/surfstat.f90:891-907); device buffers
 // [nfield][nomega][nk].

@@ -302,6 +302,15 @@ class SurfaceGF:
         if f.ndim == 2:
             f = f[None]
         nfield, nkx, nky = f.shape
+        if max(m1, m2) <= 2048:
+            # the sum is the same with the axes exchanged, and so is its result:
+            # no transposes (the library limits the length of its rows)
+            buf = np.ascontiguousarray(f)
+            out = np.empty((nkx, nky), dtype=np.float64)
+            self._check(self.lib.wtsurf_kplane_autocorrelation(
+                self.ctx, nky, nkx, int(m2), int(m1), nfield, _dptr(buf), _dptr(out)),
+                "wtsurf_kplane_autocorrelation")
+            return out
         buf = np.ascontiguousarray(f.transpose(0, 2, 1))
         out = np.zeros((nky, nkx), dtype=np.float64)
         self._check(self.lib.wtsurf_kplane_autocorrelation(self.ctx, nkx, nky, int(m1), int(m2),
