@@ -212,6 +212,9 @@ int wtsurf_kplane_autocorrelation(wtsurf_ctx *ctx, int nkx, int nky, int m1, int
  * Each sum is taken in the reference's order. */
 int wtsurf_kpath_jdos(wtsurf_ctx *ctx, int nk, int nomega, int nfield,
                       const double *fields, double *out);
+/* The same sums for arrays with the energy fastest, [nfield][nk][nomega]. */
+int wtsurf_kpath_jdos_energy_fastest(wtsurf_ctx *ctx, int nk, int nomega, int nfield,
+                                     const double *fields, double *out);
 
 /* Largest Ndim the FP64 decimation kernels are built for. */
 int wtsurf_max_ndim(void);

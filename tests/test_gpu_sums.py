@@ -1,5 +1,10 @@
-"""The k-plane autocorrelation at the edges of its tiles: moduli around the 8
-shifts of a thread and the row lengths where the launch shape changes."""
+"""The QPI sums at the edges of their tiles: moduli
+around the 8 shifts of a thread and the row lengths where correlate_kernel's
+launch shape changes, paths around the 8 shifts of a thread and the lengths
+where the path no longer fits the staged layouts, and both orders of
+the jdos arrays."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -43,3 +48,31 @@ def test_autocorrelation_at_row_edges(gpu, nkx, nky, m1, m2, nfield):
     # a NaN reaches every sum that has it as a term, an infinity likewise
     a[0, nkx - 1, nky - 1] = np.inf
     assert not np.isfinite(gpu.kplane_autocorrelation(a, m1, m2)).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nk", [1, 2, 7, 8, 9, 16, 17, 127, 128, 129, 602, 603, 2048, 2049, 5120, 5121])
+def test_kpath_jdos_at_path_edges(gpu, nk):
+    """Both orders of the arrays against 80-bit sums of positive terms, within
+    nk eps; energies on either side of the 16 and 4 staged at once."""
+    for nom in (1, 5, 17) if nk <= 603 else (1, 5):
+        print("path edges", nk, nom, flush=True)
+        a = np.random.default_rng(nk + nom).uniform(0.1, 1.0, (2, nk, nom))
+        h = (nk - 1) // 2
+        want = np.zeros(a.shape)
+        x = a[:, :2 * h + 1].astype(np.longdouble)
+        for iq in range(nk) if nk <= 129 else (0, 1, h - 1, h, h + 1, nk - 9, nk - 2, nk - 1):
+            s = iq + 1 - h
+            lo, hi = max(0, -s), min(2 * h, 2 * h - s)
+            if hi >= lo:
+                want[:, iq] = (x[:, lo:hi + 1] * x[:, lo + s:hi + s + 1]).sum(axis=1)
+        got = gpu.kpath_jdos(a)
+        got_k = np.zeros((2, nom, nk))
+        src = np.ascontiguousarray(a.transpose(0, 2, 1))
+        p = lambda v: v.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+        assert gpu.lib.wtsurf_kpath_jdos(gpu.ctx, nk, nom, 2, p(src), p(got_k)) == 0
+        assert np.array_equal(got, got_k.transpose(0, 2, 1))
+        nz = want > 0
+        assert np.all(np.abs(got[nz] / want[nz] - 1) <= nk * EPS)
+        if nk <= 129:
+            assert np.all(got[~nz] == 0)

@@ -31,7 +31,13 @@
 //
 //   out(iq, j) = sum_{ik = max(1, 1 - s)}^{min(2h + 1, 2h + 1 - s)} a(ik, j) a(ik + s, j)
 //
-// one thread per (iq, j, field), the terms added in the reference's order.
+// the terms added in the reference's order.  kpath_jdos_kernel stages JT
+// energies of the path in LDS and gives each thread one energy and eight
+// consecutive shifts, sliding an 8-wide window over the path: two LDS reads for
+// eight multiply-adds (one thread per sum from global memory: 388 us at 512 x
+// 512 and four fields, 50 us staged), and the same kernel reads either order of the arrays
+// (k or energy fastest), so that no caller transposes.  Paths too long for LDS take kpath_jdos_long_kernel,
+// one thread per (iq, j, field) from global memory.
 #include <algorithm>
 
 #include "wtsurf_device.h"
@@ -174,36 +180,130 @@ __global__ void __launch_bounds__(kCorrBlock) expand_kernel(const double *__rest
     }
 }
 
-// out_f(iq, j), fields and out [nfield][nomega][nk]; thread iq of row (j, f).
+// out_f(iq, j) for JT energies j of one field and 8 kCorrBlock / JT shifts iq;
+// element (f, j, ik) at f fs + j js + ik ks.  Dynamic LDS nk (JT + 1) doubles.
+template <int JT>
 __global__ void __launch_bounds__(kCorrBlock) kpath_jdos_kernel(const double *__restrict__ a,
-                                                                int nk, double *__restrict__ out) {
-    const int iq = blockIdx.x * kCorrBlock + threadIdx.x;  // 0-based
+                                                                int nk, int nomega, size_t fs,
+                                                                size_t js, size_t ks,
+                                                                double *__restrict__ out) {
+    extern __shared__ __align__(16) double lds[];  // [nk][JT + 1]
+    constexpr int LD = JT + 1;
+    const int tid = threadIdx.x;
+    const int nj = (nomega + JT - 1) / JT;
+    const int f = blockIdx.x / nj, j0 = (blockIdx.x % nj) * JT;
+    const double *src = a + f * fs + j0 * js;
+    // the faster of the two indices along the threads
+    if (ks == 1) {
+        for (int j = 0; j < JT && j0 + j < nomega; ++j)
+            for (int ik = tid; ik < nk; ik += kCorrBlock) lds[ik * LD + j] = src[j * js + ik];
+    } else {
+        for (int e = tid; e < nk * JT; e += kCorrBlock) {
+            const int j = e % JT, ik = e / JT;
+            if (j0 + j < nomega) lds[ik * LD + j] = src[j * js + ik * ks];
+        }
+    }
+    __syncthreads();
+    const int j = tid % JT, h = (nk - 1) / 2;
+    const int iq0 = 8 * (blockIdx.y * (kCorrBlock / JT) + tid / JT);
+    if (j0 + j >= nomega || iq0 >= nk) return;
+    const double *r = lds + j;
+    double acc[8], w[8];
+    int lo[8], hi[8], first = nk, last = -1, from = 0, to = nk;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int sft = iq0 + i + 1 - h;
+        lo[i] = sft < 0 ? -sft : 0;                 // 0-based first ik
+        hi[i] = sft > 0 ? 2 * h - sft : 2 * h;      // 0-based last ik
+        if (iq0 + i >= nk) hi[i] = lo[i] - 1;       // no such shift
+        acc[i] = 0.0;
+        if (hi[i] >= lo[i]) {
+            first = min(first, lo[i]);
+            last = max(last, hi[i]);
+        }
+        from = max(from, lo[i]);
+        to = min(to, hi[i]);
+    }
+    const int s0 = iq0 + 1 - h;
+    // the ends of the path, where not every shift has a term
+    auto edge = [&](int ik) {
+        const double x = r[ik * LD];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (ik >= lo[i] && ik <= hi[i]) acc[i] = fma(x, r[(ik + s0 + i) * LD], acc[i]);
+    };
+    int ik = first;
+    for (; ik < from && ik <= last; ++ik) edge(ik);
+    if (ik + 7 <= to) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = r[(ik + s0 + i) * LD];
+        for (; ik + 7 <= to; ik += 8) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const double x = r[(ik + t) * LD];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) acc[i] = fma(x, w[(t + i) & 7], acc[i]);
+                // the window's next value, past the path after its last use
+                const int n = ik + t + s0 + 8;
+                w[t] = r[(n < nk ? n : nk - 1) * LD];
+            }
+        }
+    }
+    for (; ik <= last; ++ik) edge(ik);
+    double *dst = out + f * fs + (j0 + j) * js;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if (iq0 + i < nk) dst[(iq0 + i) * ks] = acc[i];
+}
+
+// out_f(iq, j), element (f, j, ik) as above; thread iq of row (j, f).
+__global__ void __launch_bounds__(kCorrBlock) kpath_jdos_long_kernel(const double *__restrict__ a,
+                                                                     int nk, int nomega, size_t fs,
+                                                                     size_t js, size_t ks,
+                                                                     double *__restrict__ out) {
+    const int iq = blockIdx.y * kCorrBlock + threadIdx.x;  // 0-based
     if (iq >= nk) return;
-    const size_t row = (size_t)blockIdx.y * nk;
+    const size_t row = (blockIdx.x / nomega) * fs + (blockIdx.x % nomega) * js;
     const double *r = a + row;
     const int h = (nk - 1) / 2;
     const int sft = iq + 1 - h;
     const int lo = sft < 0 ? -sft : 0;                       // 0-based first ik
     const int hi = sft > 0 ? 2 * h - sft : 2 * h;            // 0-based last ik
     double s = 0.0;
-    for (int ik = lo; ik <= hi; ++ik) s += r[ik] * r[ik + sft];
-    out[row + iq] = s;
+    for (int ik = lo; ik <= hi; ++ik) s += r[ik * ks] * r[(ik + sft) * ks];
+    out[row + iq * ks] = s;
 }
 
 }  // namespace
 
 int kplane_corr_max_m() { return kKplaneMaxM; }
 
-int kpath_jdos_launch(const double *fields, int nk, int nomega, int nfield, double *out,
-                      hipStream_t s) {
+int kpath_jdos_launch(const double *fields, int nk, int nomega, int nfield, bool k_fastest,
+                      double *out, hipStream_t s) {
     if (nk < 1 || nomega < 1 || nfield < 1 || (long)nomega * nfield > 65535L * 1024) return -1;
-    const long rows = (long)nomega * nfield;
-    for (long r0 = 0; r0 < rows; r0 += 65535) {
-        const int nr = (int)std::min<long>(rows - r0, 65535);
-        hipLaunchKernelGGL(kpath_jdos_kernel, dim3((nk + kCorrBlock - 1) / kCorrBlock, nr),
-                           dim3(kCorrBlock), 0, s, fields + (size_t)r0 * nk, nk,
-                           out + (size_t)r0 * nk);
-    }
+    const size_t fs = (size_t)nk * nomega, js = k_fastest ? nk : 1, ks = k_fastest ? 1 : nomega;
+    auto go = [&](auto kernel, int JT) {
+        const size_t lds = (size_t)nk * (JT + 1) * sizeof(double);
+        if (lds > (size_t)64 * 1024 &&
+            hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            (void)hipGetLastError();  // the launch reports whether the size is accepted
+        const int per = 8 * kCorrBlock / JT;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nfield * ((nomega + JT - 1) / JT), (nk + per - 1) / per),
+                           dim3(kCorrBlock), lds, s, fields, nk, nomega, fs, js, ks, out);
+    };
+    // as many energies as keep two workgroups of LDS on a CU
+    constexpr int kMaxLds = 80 * 1024 / sizeof(double);
+    if (nk <= kMaxLds / 17)
+        go(kpath_jdos_kernel<16>, 16);
+    else if (nk <= kMaxLds / 5)
+        go(kpath_jdos_kernel<4>, 4);
+    else if (nk <= kMaxLds / 2)
+        go(kpath_jdos_kernel<1>, 1);
+    else
+        hipLaunchKernelGGL(kpath_jdos_long_kernel,
+                           dim3((unsigned)nfield * nomega, (nk + kCorrBlock - 1) / kCorrBlock),
+                           dim3(kCorrBlock), 0, s, fields, nk, nomega, fs, js, ks, out);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

@@ -148,8 +148,8 @@ int kplane_corr_max_m();
 size_t kplane_corr_doubles(int m1, int m2, int nfield);
 int kplane_corr_launch(const KplaneCorrArgs &k, hipStream_t s);
 // k-path joint density of states (src/surfstat.f90:891-907); device buffers
-// [nfield][nomega][nk].
-int kpath_jdos_launch(const double *fields, int nk, int nomega, int nfield, double *out,
-                      hipStream_t s);
+// [nfield][nomega][nk] (k_fastest) or [nfield][nk][nomega].
+int kpath_jdos_launch(const double *fields, int nk, int nomega, int nfield, bool k_fastest,
+                      double *out, hipStream_t s);
 
 }  // namespace wtsurf

@@ -75,6 +75,8 @@ SIGNATURES = {
     "wtsurf_kplane_autocorrelation": (ctypes.c_int, [ctypes.c_void_p] + [ctypes.c_int] * 5
                                       + [_dp, _dp]),
     "wtsurf_kpath_jdos": (ctypes.c_int, [ctypes.c_void_p] + [ctypes.c_int] * 3 + [_dp, _dp]),
+    "wtsurf_kpath_jdos_energy_fastest": (ctypes.c_int, [ctypes.c_void_p] + [ctypes.c_int] * 3
+                                         + [_dp, _dp]),
     "wtsurf_max_ndim": (ctypes.c_int, []),
 }
 
@@ -327,11 +329,11 @@ class SurfaceGF:
         if single:
             f = f[None]
         nfield, nk, nom = f.shape
-        buf = np.ascontiguousarray(f.transpose(0, 2, 1))
-        out = np.zeros_like(buf)
-        self._check(self.lib.wtsurf_kpath_jdos(self.ctx, nk, nom, nfield, _dptr(buf), _dptr(out)),
-                    "wtsurf_kpath_jdos")
-        out = out.transpose(0, 2, 1).copy()
+        buf = np.ascontiguousarray(f)
+        out = np.empty_like(buf)
+        self._check(self.lib.wtsurf_kpath_jdos_energy_fastest(self.ctx, nk, nom, nfield, _dptr(buf),
+                                                              _dptr(out)),
+                    "wtsurf_kpath_jdos_energy_fastest")
         return out[0] if single else out
 
     # ---- resident split (inputs stay in device memory) -------------------
