@@ -1,12 +1,14 @@
-"""The QPI sums at the edges of their tiles: moduli
+"""The QPI sums and the H00/H01 download at the edges of their tiles: moduli
 around the 8 shifts of a thread and the row lengths where correlate_kernel's
 launch shape changes, paths around the 8 shifts of a thread and the lengths
-where the path no longer fits the staged layouts, and both orders of
-the jdos arrays."""
+where the path no longer fits the staged layouts, both orders of the jdos
+arrays, and more k points than one piece of the download holds."""
 import ctypes
 
 import numpy as np
 import pytest
+
+from wannier_tools_amd import model as M
 
 EPS = np.finfo(np.float64).eps
 
@@ -76,3 +78,19 @@ def test_kpath_jdos_at_path_edges(gpu, nk):
         assert np.all(np.abs(got[nz] / want[nz] - 1) <= nk * EPS)
         if nk <= 129:
             assert np.all(got[~nz] == 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,nk", [(3, 70), (16, 5), (200, 110)])
+def test_ham_of_many_k_points(gpu, n, nk):
+    """A whole list of k points (at n = 200 more than one piece of 64 MiB)
+    against the points one by one, bit for bit."""
+    print("ham", n, nk, flush=True)
+    irvec, hr = M.synthetic_model(n, 1, 0.4, M.decay_l2(1.5), seed=n).surface_cell()
+    gpu.set_model_arrays(n, 1, irvec, hr)
+    k = np.random.default_rng(n).uniform(-0.5, 0.5, (nk, 2))
+    h00, h01 = gpu.ham_qlayer2qlayer(k)
+    assert h00.shape == h01.shape == (nk, n, n)
+    for i in (0, 1, nk // 2, nk - 7 if nk > 7 else 0, nk - 1):
+        a, b = gpu.ham_qlayer2qlayer(k[i])
+        assert np.array_equal(a, h00[i]) and np.array_equal(b, h01[i])

@@ -12,6 +12,8 @@
 // is one workgroup per (k, slot): each thread owns Hij(d) elements, sums over
 // the slot's R and scatters the result to every H00/H01 block using that
 // slot, writing the NP x NP padded layout the decimation kernel reads.
+#include <algorithm>
+
 #include "wtsurf_device.h"
 #include "wtsurf_internal.h"
 
@@ -60,6 +62,26 @@ __global__ void hij_scatter_kernel(FourierArgs a) {
             dst[(nw * (i - 1) + rr) + (size_t)(nw * (jb - 1) + cc) * NP] = acc;
         }
     }
+}
+
+__global__ void unpad_kernel(const double2 *__restrict__ hk, long total, int n, int NP,
+                             double2 *__restrict__ h00, double2 *__restrict__ h01) {
+    const int nn = n * n;
+    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total;
+         e += (long)gridDim.x * blockDim.x) {
+        const long ik = e / nn;
+        const int r = (int)(e - ik * nn), i = r % n, j = r / n;
+        const double2 *h = hk + (size_t)ik * 2 * NP * NP + i + (size_t)j * NP;
+        h00[e] = h[0];
+        h01[e] = h[(size_t)NP * NP];
+    }
+}
+
+int unpad_launch(const double2 *hk, int nk, int n, int NP, double2 *h00, double2 *h01, hipStream_t s) {
+    const long total = (long)nk * n * n;
+    const unsigned blocks = (unsigned)std::min<long>((total + 255) / 256, 1 << 16);
+    hipLaunchKernelGGL(unpad_kernel, dim3(blocks), dim3(256), 0, s, hk, total, n, NP, h00, h01);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int fourier_launch(const FourierArgs &a, hipStream_t s) {

@@ -136,7 +136,7 @@ struct wtsurf_ctx {
     // grid
     int nk = 0, nomega = 0;
     DevBuf<double> kpts, omega;
-    DevBuf<double2> phase, hk;
+    DevBuf<double2> phase, hk, hpack;
     DevBuf<double> qpi;  // fields, scratch and result of the QPI sums
     DevBuf<double> dos_l, dos_r, dos_b;
     DevBuf<int> iters, status;
@@ -282,7 +282,7 @@ void wtsurf_ctx_destroy(wtsurf_ctx *c) {
     c->hr.release(); c->irvec.release(); c->slot_begin.release();
     c->d_top.release(); c->d_bot.release();
     c->kpts.release(); c->omega.release(); c->phase.release(); c->hk.release();
-    c->qpi.release();
+    c->hpack.release(); c->qpi.release();
     c->dos_l.release(); c->dos_r.release(); c->dos_b.release();
     c->inst_k.release(); c->inst_w.release(); c->inst_eta.release(); c->spin.release();
     c->iters.release(); c->status.release(); c->work.release(); c->state.release();
@@ -420,18 +420,22 @@ int wtsurf_ham_qlayer2qlayer(wtsurf_ctx *c, int nk, const double *kpts, double *
     c->nomega = 0;
     if (int r = run_fourier(c)) return r;
     const int n = c->n, NP = 16 * padded_q(n);
-    WT_HIP(c, hipStreamSynchronize(c->stream));
-    std::vector<double2> buf((size_t)2 * NP * NP);
-    for (int ik = 0; ik < nk; ++ik) {
-        WT_HIP(c, hipMemcpy(buf.data(), c->hk.p + (size_t)ik * 2 * NP * NP,
-                            buf.size() * sizeof(double2), hipMemcpyDeviceToHost));
-        for (int m = 0; m < 2; ++m) {
-            double *dst = (m == 0 ? h00 : h01) + 2 * (size_t)ik * n * n;
-            for (int j = 0; j < n; ++j)
-                std::memcpy(dst + 2 * (size_t)j * n, &buf[(size_t)m * NP * NP + (size_t)j * NP],
-                            n * sizeof(double2));
-        }
+    // the pads come off on the device, and whole arrays go to the caller in
+    // pieces of at most 64 MiB
+    const size_t nn = (size_t)n * n;
+    const int step = (int)std::min<size_t>(nk, std::max<size_t>(1, ((size_t)64 << 20) / (nn * sizeof(double2))));
+    if (c->hpack.ensure(2 * step * nn)) return c->fail("out of device memory (H00, H01)");
+    for (int ik = 0; ik < nk; ik += step) {
+        const int m = std::min(step, nk - ik);
+        double2 *p0 = c->hpack.p, *p1 = p0 + m * nn;
+        if (unpad_launch(c->hk.p + (size_t)ik * 2 * NP * NP, m, n, NP, p0, p1, c->stream))
+            return c->fail("H00/H01 unpadding launch failed");
+        WT_HIP(c, hipMemcpyAsync(h00 + 2 * ik * nn, p0, m * nn * sizeof(double2),
+                                 hipMemcpyDeviceToHost, c->stream));
+        WT_HIP(c, hipMemcpyAsync(h01 + 2 * ik * nn, p1, m * nn * sizeof(double2),
+                                 hipMemcpyDeviceToHost, c->stream));
     }
+    WT_HIP(c, hipStreamSynchronize(c->stream));
     c->nk = 0;  // hk no longer matches an uploaded grid
     return 0;
 }

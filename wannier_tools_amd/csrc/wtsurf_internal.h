@@ -134,6 +134,8 @@ struct FourierArgs {
     int NP;
 };
 int fourier_launch(const FourierArgs &a, hipStream_t s);
+// hk [nk][2][NP*NP] without its pads: h00 and h01 [nk][n*n].
+int unpad_launch(const double2 *hk, int nk, int n, int NP, double2 *h00, double2 *h01, hipStream_t s);
 
 // QPI autocorrelation over a k-plane (src/fermiarc.f90:496-560), device buffers.
 constexpr int kKplaneMaxM = 2048;  // largest m1 (rows in LDS)
