@@ -19,7 +19,7 @@ LIB = os.path.join(HERE, "libwtsurf.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-SOURCES = ["decimate.hip", "mid.hip", "small.hip", "fourier.hip", "qpi.hip", "wtsurf_cabi.hip"]
+SOURCES = ["decimate.hip", "mid.hip", "small.hip", "tiny.hip", "fourier.hip", "qpi.hip", "wtsurf_cabi.hip"]
 HIPFLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

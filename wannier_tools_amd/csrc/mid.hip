@@ -18,7 +18,6 @@
 // memory between rounds and takes the next (k, omega) instance from a device
 // counter once its previous one has converged.
 #include <algorithm>
-#include <type_traits>
 #include <utility>
 
 #include "decimate_common.h"
@@ -69,19 +68,6 @@ struct MidSlot {
 };
 
 enum : int { kMidEmpty = 0, kMidLoop = 1, kMidDone = 2 };
-
-// sqrt(x^2 + y^2) scaled by the exponent of the larger part, so that the
-// squares neither overflow nor underflow.
-__device__ __forceinline__ double cabs_scaled(double x, double y) {
-    const int e = __builtin_amdgcn_frexp_exp(fmax(fabs(x), fabs(y)));
-    const double xs = __builtin_amdgcn_ldexp(x, -e), ys = __builtin_amdgcn_ldexp(y, -e);
-    return __builtin_amdgcn_ldexp(sqrt(fma(xs, xs, ys * ys)), e);
-}
-
-// D += -A B: the FP64 MFMA's negate bit of the first operand.
-__device__ __forceinline__ v4d mfma_neg(double a, double b, v4d c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 1);
-}
 
 // The element at a byte offset from a uniform base: base in scalar registers,
 // offset in one vector register.
@@ -288,42 +274,11 @@ struct MidGjShared {
     double2 diag[NB], part[NB];   // final inverses: G(i, i), G(i, spin partner)
 };
 
-// Spin partner of orbital i (0-based) in layers of nw orbitals (-1: none), and
-// whether i is spin up.
-__device__ __forceinline__ int spin_partner(int i, int nw, bool &up) {
-    const int nh = nw / 2, l = i % nw;
-    up = l < nh;
-    return l >= 2 * nh ? -1 : up ? i + nh : i - nh;
-}
-
 // A wave's role (0 .. W - 1: columns, W: panels), another one for the same
 // SIMD in every other workgroup.
 template <int KT>
 __device__ __forceinline__ int mid_wave(int tid) {
     return (uniform(tid >> 6) + (int)blockIdx.x) % (MidGj<KT>::W + 1);
-}
-
-// 1/z as crecip_fast, the binary exponent e of |re| + |im| given: the scaled
-// |z|^2 lies in [1/8, 1).
-__device__ __forceinline__ double2 crecip_scaled(double2 z, int e) {
-    const double x = __builtin_amdgcn_ldexp(z.x, -e), y = __builtin_amdgcn_ldexp(z.y, -e);
-    const double d = fma(x, x, y * y);
-    double r = __builtin_amdgcn_rcp(d);
-    r = fma(r, fma(-d, r, 1.0), r);
-    r = fma(r, fma(-d, r, 1.0), r);
-    return make_double2(__builtin_amdgcn_ldexp(x * r, -e), __builtin_amdgcn_ldexp(-y * r, -e));
-}
-
-// LDS written by some lanes of a wave is read by others of the same wave
-// after this: the LDS keeps a wave's accesses in order, the compiler must too.
-__device__ __forceinline__ void wave_order() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-template <int... J, typename F>
-__device__ __forceinline__ void each_of(std::integer_sequence<int, J...>, F &&step) {
-    (step(std::integral_constant<int, J>()), ...);
 }
 
 // d of lane 8 a + k to every lane 8 a + b (two DPP row broadcasts, one for each

@@ -1,9 +1,10 @@
-// Decimation for small orders (Ndim <= 32) on the vector ALUs, one workgroup
-// per instance for its whole decimation (src/surfgreen.f90:74-134).
+// Decimation for orders 17 to 32 on the vector ALUs, one workgroup per
+// instance for its whole decimation (src/surfgreen.f90:74-134); smaller orders
+// are tiny.hip's.
 //
-// At these orders a 16 x 16 matrix-core tile wastes most of its work on
-// padding (Ndim 8: seven eighths), and the round schedule's traffic of the
-// slot state through HBM and its launches dominate.  MI355X's FP64 vector
+// At these orders the 16 x 16 matrix-core tiles are partly padding, and the
+// round schedule's traffic of the slot state through HBM and its launches
+// weigh on it.  MI355X's FP64 vector
 // rate equals its FP64 matrix rate, so here every product is a plain FMA
 // loop over the true order n.  Each instance lives in one workgroup of W
 // waves from its set-up to its traces: its matrices in LDS, eps_s, eps_t and
@@ -95,58 +96,38 @@ __device__ __forceinline__ bool small_gj(double2 (&x)[E], int n,
             if (c >= n) break;
             int p;
             double2 r, m;
-            if constexpr (W == 1) {
-                // one wave: the pivot, 1/pivot and the multipliers by
-                // cross-lane moves, with no LDS exchange or barrier
+            const int b = c & 1;
+            if (wave == jh / GPW) {
                 const double v = (jc == jh && fr) ? fabs(x[t].x) + fabs(x[t].y) : -1.0;
-                // the column's lanes lie in one DPP row (NP <= 16): a row maximum
-                const double best = NP <= 16 ? row_max_f64(v, (NP * jh) >> 4) : wave_max_f64(v);
+                const double best = wave_max_f64(v);
                 if (!(best > 0.0)) {
-                    singular = true;
-                    break;
-                }
-                const unsigned long long msk = __ballot(v == best);
-                const int pl = uniform(__ffsll((long long)msk) - 1);
-                p = pl - NP * jh;
-                const double2 piv = make_double2(readlane_f64(x[t].x, pl), readlane_f64(x[t].y, pl));
-                r = crecip_fast(piv);
-                const int hl = i + NP * jh;  // lane holding X[i][c]
-                m = cmul(make_double2(__shfl(x[t].x, hl), __shfl(x[t].y, hl)), r);
-                if (i == p) m = make_double2(0.0, 0.0);
-            } else {
-                const int b = c & 1;
-                if (wave == jh / GPW) {
-                    const double v = (jc == jh && fr) ? fabs(x[t].x) + fabs(x[t].y) : -1.0;
-                    const double best = wave_max_f64(v);
-                    if (!(best > 0.0)) {
-                        if (lane == 0) sh.sing[b] = 1;
-                    } else {
-                        const unsigned long long msk = __ballot(v == best);
-                        const int pl = uniform(__ffsll((long long)msk) - 1);
-                        const int ph = pl - NP * (jh % GPW);
-                        const double2 piv = make_double2(readlane_f64(x[t].x, pl), readlane_f64(x[t].y, pl));
-                        const double2 rh = crecip_fast(piv);
-                        if (jc == jh) {
-                            double2 mh = cmul(x[t], rh);
-                            if (i == ph) mh = make_double2(0.0, 0.0);
-                            sh.mcol[b][i] = mh;
-                        }
-                        if (lane == 0) {
-                            sh.piv[b] = ph;
-                            sh.rr[b] = rh;
-                            sh.sing[b] = 0;
-                        }
+                    if (lane == 0) sh.sing[b] = 1;
+                } else {
+                    const unsigned long long msk = __ballot(v == best);
+                    const int pl = uniform(__ffsll((long long)msk) - 1);
+                    const int ph = pl - NP * (jh % GPW);
+                    const double2 piv = make_double2(readlane_f64(x[t].x, pl), readlane_f64(x[t].y, pl));
+                    const double2 rh = crecip_fast(piv);
+                    if (jc == jh) {
+                        double2 mh = cmul(x[t], rh);
+                        if (i == ph) mh = make_double2(0.0, 0.0);
+                        sh.mcol[b][i] = mh;
+                    }
+                    if (lane == 0) {
+                        sh.piv[b] = ph;
+                        sh.rr[b] = rh;
+                        sh.sing[b] = 0;
                     }
                 }
-                __syncthreads();
-                if (uniform(sh.sing[b])) {
-                    singular = true;
-                    break;
-                }
-                p = uniform(sh.piv[b]);
-                r = sh.rr[b];
-                m = sh.mcol[b][i];
             }
+            __syncthreads();
+            if (uniform(sh.sing[b])) {
+                singular = true;
+                break;
+            }
+            p = uniform(sh.piv[b]);
+            r = sh.rr[b];
+            m = sh.mcol[b][i];
             const int src = p + NP * (jc % GPW);  // lane of (p, jc) in this wave
 #pragma unroll
             for (int u = 0; u < EPL; ++u) {
@@ -381,8 +362,7 @@ int decimate_small_max_n() { return 32; }
 int decimate_small_run(const DecimateArgs &a, int num_cu, hipStream_t s) {
     if (a.n < 1 || a.n > decimate_small_max_n() || num_cu < 1) return -1;
     if (hipMemsetAsync(a.queue, 0, 2 * sizeof(unsigned), s) != hipSuccess) return -1;
-    if (a.n <= 8) return launch_small<8, 1>(a, num_cu, s);
-    if (a.n <= 16) return launch_small<16, 1>(a, num_cu, s);
+    if (a.n <= decimate_tiny_max_n()) return decimate_tiny_run(a, num_cu, s);
     return launch_small<32, 8>(a, num_cu, s);
 }
 

@@ -95,6 +95,9 @@ int decimate_persistent_run(const DecimateArgs &a, int q, int precision, int nbl
 // a.state unused).  Returns once the launch is queued on s.
 int decimate_small_max_n();
 int decimate_small_run(const DecimateArgs &a, int num_cu, hipStream_t s);
+// The same up to decimate_tiny_max_n(), in the registers of one wave (tiny.hip).
+int decimate_tiny_max_n();
+int decimate_tiny_run(const DecimateArgs &a, int num_cu, hipStream_t s);
 
 // FP64 orders up to decimate_mid_max_n() as rounds of two kernels with the
 // inverse in registers (mid.hip).  State of one slot between rounds; two per
