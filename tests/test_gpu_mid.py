@@ -1,4 +1,4 @@
-"""The FP64 rounds of orders up to 80 (inverse in registers, wave-strip GEMMs)
+"""The FP64 rounds of orders up to 112 (inverse in registers, wave-strip GEMMs)
 against the oracle where their tiling can go wrong: orders on either side of
 every multiple of 8, a single instance (whose products are split over the
 chip) against the same instance in a grid, more instances than slots, singular
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n", [1, 7, 8, 9, 17, 25, 33, 40, 41, 48, 49, 56, 57, 64, 65, 71, 72, 73,
-                               79, 80])
+                               79, 80, 81, 88, 89, 96, 97, 104, 105, 112, 113])
 def test_orders_around_multiples_of_8(gpu, oracle_lib, n):
     print("mid order", n, flush=True)
     irvec, hr = M.synthetic_model(n, 1, 0.4, M.decay_l2(1.5), seed=600 + n).surface_cell()
@@ -54,7 +54,8 @@ def test_more_instances_than_slots(gpu):
             assert np.array_equal(a[:, :60], a[:, 60 * r:60 * (r + 1)])
 
 
-@pytest.mark.parametrize("n,c", [(40, 0), (72, 23), (72, 71), (77, 76), (80, 40)])
+@pytest.mark.parametrize("n,c", [(40, 0), (72, 23), (72, 71), (77, 76), (80, 40), (81, 80),
+                                 (108, 50), (112, 111)])
 def test_zero_and_nan_pivot_columns(gpu, n, c):
     """Column c of omega - H00 exactly zero (eta = 0), or all NaN: every inverse
     is the identity, as the reference's inv leaves it."""

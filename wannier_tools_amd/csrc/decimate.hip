@@ -1,6 +1,6 @@
 // Batched Lopez-Sancho decimation on gfx950: the FP32-with-FP64-accumulation
 // rounds and the persistent schedules up to order 80, and the FP64 rounds
-// beyond (the FP64 rounds up to order 80 are in mid.hip).
+// beyond order 112 (the FP64 rounds up to there are in mid.hip).
 //
 // Restates surfgreen_1985 (src/surfgreen.f90:74-134) for many (k, omega)
 // instances.  Per iteration:
@@ -1905,9 +1905,9 @@ int decimate_max_q() { return kMaxQ; }
 
 template <int Q, typename R>
 static int launch_round(const DecimateArgs &a, int per_set, int set, bool gj, hipStream_t s) {
-    if constexpr ((Q > 5) == std::is_same_v<R, float>) {
+    if constexpr (std::is_same_v<R, float> ? Q > 5 : Q <= 7) {
         // no FP32 kernels beyond order 80 (the C ABI refuses that case); FP64
-        // rounds up to order 80 are mid.hip's
+        // rounds up to order 112 are mid.hip's
         return -1;
     } else if constexpr (Q <= 5) {
         constexpr size_t gj_lds = GjLay<Q, R>::bytes;
@@ -1967,7 +1967,7 @@ static void allow_lds() {
     if constexpr (Q <= 5 && std::is_same_v<R, float>)
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gj_round_kernel<Q, R>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)GjLay<Q, R>::bytes);
-    else if constexpr (Q > 5 && std::is_same_v<R, double>)
+    else if constexpr (Q > 7 && std::is_same_v<R, double>)
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gj_large_round_kernel<Q, R>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)GjLayL<Q>::bytes);
     else

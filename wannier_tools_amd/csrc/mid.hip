@@ -1,4 +1,4 @@
-// FP64 decimation for orders up to 80 as rounds of two kernels
+// FP64 decimation for orders up to 112 as rounds of two kernels
 // (src/surfgreen.f90:74-134 over many instances).  An iteration is
 //
 //   g = (z - eps_i)^-1                                       mid_inverse_kernel
@@ -50,7 +50,7 @@ struct MidLay {
         return ((c >> 4) * KS + (k >> 2)) * 64 + (c & 15) + 16 * (k & 3);
     }
 };
-static_assert(MidLay<10>::stride <= kMidMaxSlotBytes, "slot larger than its host-side bound");
+static_assert(MidLay<10>::stride <= kMidNoallocSlotBytes, "slot larger than its host-side bound");
 
 template <int KT>
 struct MidSlot {
@@ -92,7 +92,7 @@ __device__ __forceinline__ double2 frag_at(const double2 *base, unsigned off) {
 // product, m^T, are then laid out exactly as the B operand of the second, and
 // m1, m2 never leave the registers.
 template <int KT>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KT <= 10 ? 3 : 2)))
 mid_gemm_kernel(void *work, const MidState *__restrict__ state, int slots, int csplit) {
     using L = MidLay<KT>;
     using P = Prec<double>;
@@ -168,7 +168,8 @@ mid_gemm_kernel(void *work, const MidState *__restrict__ state, int slots, int c
 
     // the second product, one 16-column tile of [alpha beta] at a time; a
     // fragment register is loaded again right after its use, GS steps ahead
-    constexpr int GS = KT % 3 == 0 ? 6 : KT % 5 == 0 ? 5 : KT % 7 == 0 ? 7 : KT % 2 == 0 ? 4 : 2;
+    constexpr int GS = KT % 3 == 0 ? 6 : KT % 5 == 0 ? 5 : KT % 7 == 0 ? 7
+                     : KT == 11 || KT == 13 ? KT : KT % 2 == 0 ? 4 : 2;
     constexpr int NG = KS / GS;
     static_assert(NG * GS == KS, "whole groups");
     const double2 *col = AB + t0 * (KS * 64);
@@ -228,7 +229,7 @@ mid_gemm_kernel(void *work, const MidState *__restrict__ state, int slots, int c
 
 // ---------------------------------------------------------------------------
 // Gauss-Jordan inverses, one workgroup each, the matrix in the registers of
-// W = 3 waves: lane (a = lane % 8, b = lane / 8) of wave w holds rows a + 8 s
+// W waves (3 up to order 80, 7 beyond): lane (a = lane % 8, b = lane / 8) of wave w holds rows a + 8 s
 // (s < KT) of columns 8 (w + W t) + b (t < CL).  Partial pivoting on
 // |re| + |im| over the rows not yet used (the izamax rule of zgesv up to
 // 2^-13 of the value), rows never swapped: step c's pivot row p keeps its
@@ -237,10 +238,10 @@ mid_gemm_kernel(void *work, const MidState *__restrict__ state, int slots, int c
 // is then X^-1[step of r][pivot row of step c].
 //
 // Columns are eliminated in panels of 8, one register group t of one wave, by
-// a fourth wave: it takes the panel from LDS, runs its steps by itself and
+// one more wave: it takes the panel from LDS, runs its steps by itself and
 // publishes the panel's columns M.  The others then take the pivot rows T of their own columns out of their
 // registers and add M T, on the vector ALUs, whose FP64 rate is that of the
-// matrix cores: the group of the next panel first, which the fourth wave then
+// matrix cores: the group of the next panel first, which that wave then
 // eliminates while they update the rest.
 //
 // What it is bound by: an inverse alone is a chain of n pivot searches and
@@ -251,12 +252,13 @@ struct MidGj {
     // Four waves a workgroup: those of three or five leave SIMDs idle (the
     // dispatcher refills them badly: 2048 workgroups of three waves take 1141
     // us where 1024 of four take 760 us).
-    static constexpr int W = 3;
+    // Eight where the matrix needs the registers of two waves a SIMD.
+    static constexpr int W = KT <= 10 ? 3 : 7;
     static constexpr int CL = (KT + W - 1) / W;  // column groups of the first waves
     static constexpr int NT = 64 * (W + 1);
     static constexpr int LDM = 8 * KT + (KT % 2 ? 0 : 8);  // columns on alternate halves of the banks
     // waves per SIMD that the registers are capped for
-    static constexpr int OCC = KT * CL <= 16 ? 4 : KT * CL <= 30 ? 3 : 2;
+    static constexpr int OCC = W == 7 ? 2 : KT * CL <= 16 ? 4 : KT * CL <= 30 ? 3 : 2;
 };
 
 template <int KT>
@@ -821,7 +823,8 @@ int launch_mid(const DecimateArgs &a, MidState *in, MidState *out, void *work, i
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-#define WTSURF_FOR_EACH_KT(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10)
+#define WTSURF_FOR_EACH_KT(X) \
+    X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14)
 
 int dispatch_mid(int kt, const DecimateArgs &a, MidState *in, MidState *out, void *work, int slots,
                  int csplit, bool inverse, hipStream_t s) {
@@ -842,7 +845,12 @@ constexpr int kMidRoundsPerBatch = 4;
 
 }  // namespace
 
-int decimate_mid_max_n() { return 80; }
+// Beyond 112 the inverse's registers (28 complex of a lane at two waves a SIMD)
+// run out.  Between 81 and 112 the kernels with the matrix in global memory that
+// took these orders before: 1500 instances of order 108 59.6 ms, 47.0 here;
+// 400 of order 96 11.8 and 10.7, of order 81 11.3 and 8.7; one of order 108
+// 9.6 and 4.6.
+int decimate_mid_max_n() { return 112; }
 
 size_t decimate_mid_slot_bytes(int n) {
     switch ((n + 7) / 8) {

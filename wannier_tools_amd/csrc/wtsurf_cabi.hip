@@ -67,7 +67,7 @@ constexpr size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign;
 constexpr size_t kOffHk = 0;
 constexpr size_t kOffWork = kOffHk + align_up((size_t)2 * kNoallocNP * kNoallocNP * sizeof(double2));
 constexpr size_t kOffState =
-    kOffWork + align_up(std::max((size_t)kSlotSets * slot_bytes_lds_fp64(kNoallocNP / 16), kMidMaxSlotBytes));
+    kOffWork + align_up(std::max((size_t)kSlotSets * slot_bytes_lds_fp64(kNoallocNP / 16), kMidNoallocSlotBytes));
 constexpr size_t kOffQueue =
     kOffState + align_up((size_t)kSlotSets * std::max(sizeof(SlotState), sizeof(MidState)));
 constexpr size_t kOffG = kOffQueue + kAlign;
@@ -206,11 +206,12 @@ static int sync_orbitals(wtsurf_ctx *c) {
     return 0;
 }
 
-// FP64 rounds of orders up to 80 (mid.hip): the schedule asked for is the
-// rounds, or automatic above the small kernel's orders.
+// FP64 rounds of mid.hip's orders: the schedule asked for is the rounds, or
+// automatic above the small kernel's orders, or has no kernel for the order.
 static bool use_mid(const wtsurf_ctx *c, int n, int precision) {
     if (precision != WTSURF_FP64 || n > decimate_mid_max_n()) return false;
-    if (c->schedule == WTSURF_SCHEDULE_PERSISTENT) return false;
+    if (c->schedule == WTSURF_SCHEDULE_PERSISTENT && padded_q(n) <= decimate_persistent_max_q())
+        return false;
     return c->schedule == WTSURF_SCHEDULE_ROUNDS || n > decimate_small_max_n();
 }
 

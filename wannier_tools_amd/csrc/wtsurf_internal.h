@@ -113,7 +113,7 @@ struct MidState {
 struct MidPlan {
     int sets = 1, per_set = 1;  // slot sets (one stream each) and slots per set
 };
-constexpr size_t kMidMaxSlotBytes = (size_t)922112;  // slot of order 80
+constexpr size_t kMidNoallocSlotBytes = (size_t)922112;  // slot of order 80
 int decimate_mid_max_n();
 size_t decimate_mid_slot_bytes(int n);
 MidPlan decimate_mid_plan(int ninst, int num_cu);
