@@ -21,7 +21,8 @@
 // R2 rows of a_f over the row of E_f, one LDS read of a row and one of E
 // (broadcast) for 8 R2 multiply-adds, where a thread per (p1, p2) took two
 // reads for each: at 257 x 257, moduli 256 and four fields, 6.97 ms, bound by
-// the LDS reads, and 0.79 ms now.  Rows go in groups of G values of c2, one per group of
+// the LDS reads, and 0.74 ms now
+// (rows staged one load at a time a thread 0.79, windows of two rows 0.81).  Rows go in groups of G values of c2, one per group of
 // threads; the sum over c2 is cut into slices so that there are workgroups for
 // the whole chip, and expand_kernel adds the slices in order.  Bound by the
 // FP64 vector ALUs.
@@ -67,22 +68,26 @@ __global__ void __launch_bounds__(kCorrBlock) fold_kernel(const double *__restri
     }
 }
 
-// Place of element x of a row of a in LDS: one double of padding in eight, so
-// that the threads' windows (8 apart) fall on different banks.
-__device__ __forceinline__ int skew(int x) { return x + (x >> 3); }
+// Place of element x of a row of a in LDS: two doubles of padding in eight, so
+// that the threads' windows (8 apart) fall on different banks and on 16 B.
+__host__ __device__ __forceinline__ constexpr int skew(int x) { return x + 2 * (x >> 3); }
+// Length of a row of a of len elements, even.
+__host__ __device__ __forceinline__ constexpr int row_length(int len) { return (skew(len) + 2) & ~1; }
 
 // Slice blockIdx.y of C(p1, p2) for p2 = R2 blockIdx.x ..: threads tp = tid % TP
 // (p1 = 8 tp .. 8 tp + 7) of group g = tid / TP (c2 = c20 + g of each chunk).
-// part [slices][m2][m1].  Dynamic LDS: G rows of E, G + R2 - 1 skewed rows of a.
+// part [slices][m2][m1].  Dynamic LDS: G rows of E (of an even length), G + R2 - 1
+// skewed rows of a.
 template <int R2>
 __global__ void __launch_bounds__(kCorrBlock) correlate_kernel(
     const double *__restrict__ a, const double *__restrict__ e, int nkx, int nky, int m1, int m2,
     int nfield, int TP, int len, double *__restrict__ part) {
     extern __shared__ __align__(16) double lds[];
     const int G = kCorrBlock / TP;
-    const int ld = skew(len) + 1;
-    double *er = lds;               // [G][m1]
-    double *ar = lds + (size_t)G * m1;  // [G + R2 - 1][ld]
+    const int ld = row_length(len);
+    const int le = (m1 + 1) & ~1;
+    double *er = lds;                   // [G][le]
+    double *ar = lds + (size_t)G * le;  // [G + R2 - 1][ld]
     const int tid = threadIdx.x;
     const int tp = tid % TP, g = tid / TP;
     const int p20 = R2 * blockIdx.x;
@@ -100,15 +105,34 @@ __global__ void __launch_bounds__(kCorrBlock) correlate_kernel(
         const double *ef = e + ((size_t)f * m2 + c20) * m1;
         const double *af = a + (size_t)f * nkx * nky;
         __syncthreads();  // the previous rows are no longer read
-        for (int j = tid; j < ng * m1; j += kCorrBlock) er[j] = ef[j];
-        for (int row = 0; row < ng + R2 - 1; ++row) {
-            const double *src = af + (size_t)nkx * ((c20 + p20 + row) % m2);
-            for (int j = tid; j < len; j += kCorrBlock) ar[row * ld + skew(j)] = src[j % m1];
+        // (four loads in flight a thread)
+        const int p2 = (c20 + p20) % m2, rows = ng + R2 - 1;
+        for (int j = tid; j < m1; j += kCorrBlock) {
+            for (int row = 0; row < rows; row += 4) {
+                double v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    int r2 = p2 + std::min(row + u, rows - 1);
+                    r2 = r2 < m2 ? r2 : r2 % m2;
+                    v[u] = af[(size_t)nkx * r2 + j];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    for (int x = j; x < len; x += m1)  // around the torus
+                        ar[std::min(row + u, rows - 1) * ld + skew(x)] = v[u];
+            }
+            for (int row = 0; row < ng; row += 4) {
+                double v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = ef[(size_t)std::min(row + u, ng - 1) * m1 + j];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) er[std::min(row + u, ng - 1) * le + j] = v[u];
+            }
         }
         __syncthreads();
         if (g < ng) {
-            const double *eg = er + g * m1;
-            const double *w0 = ar + g * ld + 9 * tp;  // window of p2 = p20 + j: row g + j
+            const double *eg = er + g * le;
+            const double *w0 = ar + g * ld + 10 * tp;  // window of p2 = p20 + j: row g + j
             double w[R2][8];
 #pragma unroll
             for (int j = 0; j < R2; ++j)
@@ -116,19 +140,32 @@ __global__ void __launch_bounds__(kCorrBlock) correlate_kernel(
                 for (int i = 0; i < 8; ++i) w[j][i] = w0[j * ld + i];
             int c1 = 0;
             for (; c1 + 8 <= m1; c1 += 8) {
-                w0 += 9;
+                w0 += 10;
+                double2 e2[4];
 #pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const double ev = eg[c1 + t];
+                for (int t = 0; t < 4; ++t) e2[t] = *reinterpret_cast<const double2 *>(eg + c1 + 2 * t);
+#pragma unroll
+                for (int t = 0; t < 8; t += 2) {
+                    double2 nw[R2];
+#pragma unroll
+                    for (int j = 0; j < R2; ++j) nw[j] = *reinterpret_cast<const double2 *>(w0 + j * ld + t);
 #pragma unroll
                     for (int j = 0; j < R2; ++j) {
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) acc[j][i] = fma(ev, w[j][(t + i) & 7], acc[j][i]);
-                        w[j][t] = w0[j * ld + t];
+                        for (int i = 0; i < 8; ++i)
+                            acc[j][i] = fma(e2[t / 2].x, w[j][(t + i) & 7], acc[j][i]);
+                        w[j][t] = nw[j].x;
+                    }
+#pragma unroll
+                    for (int j = 0; j < R2; ++j) {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i)
+                            acc[j][i] = fma(e2[t / 2].y, w[j][(t + 1 + i) & 7], acc[j][i]);
+                        w[j][t + 1] = nw[j].y;
                     }
                 }
             }
-            w0 += 9;
+            w0 += 10;
 #pragma unroll
             for (int t = 0; t < 7; ++t)
                 if (c1 + t < m1) {
@@ -322,7 +359,7 @@ static CorrPlan corr_plan(int m1, int m2, int nfield) {
     p.len = m1 + 8 * p.tp + 8;
     const int G = kCorrBlock / p.tp;
     for (p.r2 = 4;; p.r2 /= 2) {
-        const size_t rows = (size_t)G * m1 + (size_t)(G + p.r2 - 1) * (p.len + p.len / 8 + 1);
+        const size_t rows = (size_t)G * ((m1 + 1) & ~1) + (size_t)(G + p.r2 - 1) * row_length(p.len);
         p.lds = std::max(rows, (size_t)8 * kCorrBlock) * sizeof(double);
         if (p.r2 == 1 || p.lds <= (size_t)80 * 1024) break;
     }
