@@ -1368,20 +1368,22 @@ struct GemmLayL {
 // blocks of kBI x kBJ tile pairs, one pass over K per block, the block's A0 /
 // A1 rows and B columns staged through LDS by K-chunks.  kBI kBJ = 24 pairs
 // per block, three per wave.  B is read in every pass, so O1 must not be B.
-template <int Q, typename R, int MODE>
+// Only NIB row blocks of kBI tiles from ib0 on are formed (and summed); they
+// depend on no other rows of A0 and A1.
+template <int Q, typename R, int MODE, int NIB>
 __device__ __forceinline__ double dual_gemm_blocked(unsigned char *lds, double *red,
                                                     const typename Prec<R>::C *__restrict__ A0,
                                                     const typename Prec<R>::C *__restrict__ A1,
                                                     const typename Prec<R>::C *__restrict__ B,
                                                     int kdim, typename Prec<R>::C *__restrict__ O0,
                                                     typename Prec<R>::C *__restrict__ O1,
-                                                    double2 *__restrict__ E) {
+                                                    double2 *__restrict__ E, int ib0) {
     using P = Prec<R>;
     using C = typename P::C;
     using V4 = typename P::V4;
     constexpr int NP = 16 * Q;
     constexpr int RI = 16 * kBI, CJ = 16 * kBJ;
-    constexpr int NBI = (Q + kBI - 1) / kBI, NBJ = (Q + kBJ - 1) / kBJ;
+    constexpr int NBJ = (Q + kBJ - 1) / kBJ;
     constexpr int PPW = kBI * kBJ / kWaves;
     static_assert(PPW * kWaves == kBI * kBJ, "block pairs must split evenly over the waves");
     constexpr int NA = kChunkL * RI / kBlock, NB = kChunkL * CJ / kBlock;
@@ -1398,8 +1400,8 @@ __device__ __forceinline__ double dual_gemm_blocked(unsigned char *lds, double *
     // B elements e = tid + u kBlock (kk = e % kChunkL, column e / kChunkL)
 
     double asum = 0.0;
-    for (int blk = 0; blk < NBI * NBJ; ++blk) {
-        const int i0 = kBI * (blk % NBI), j0 = kBJ * (blk / NBI);
+    for (int blk = 0; blk < NIB * NBJ; ++blk) {
+        const int i0 = kBI * (ib0 + blk % NIB), j0 = kBJ * (blk / NIB);
         const int ni = Q - i0 < kBI ? Q - i0 : kBI, nj = Q - j0 < kBJ ? Q - j0 : kBJ;
         int ti[PPW], tj[PPW];
         bool act[PPW];
@@ -1783,20 +1785,34 @@ gemm_round_kernel(DecimateArgs a, int slot0) {
     }
 }
 
-// The same for orders beyond 80, with the blocked GEMM; alpha' and beta' go to
-// the other half of the slot's alpha / beta pair (iteration parity).
-template <int Q, typename R>
-__global__ void __launch_bounds__(kBlock) gemm_large_round_kernel(DecimateArgs a, int slot0) {
+// The same for orders beyond 112, with the blocked GEMM; alpha' and beta' go to
+// the other half of the slot's alpha / beta pair (iteration parity).  A slot's
+// row blocks go to one workgroup, or (SPREAD) to one each (on one XCD, whose L2
+// then serves g, alpha and beta to all of them): the rows of all three
+// products depend on the same rows of alpha and beta only.  The last of them to
+// finish adds their parts of sum |alpha'| in order and applies the stop rule.
+// (With the share a run-time number the unspread rounds took 1% longer.)
+template <int Q, typename R, bool SPREAD>
+__global__ void __launch_bounds__(kBlock) gemm_large_round_kernel(DecimateArgs a, int slot0,
+                                                                  int slots) {
     __shared__ __align__(16) unsigned char lds[GemmLayL<Q, R>::bytes];
     __shared__ double red[kWaves];
     __shared__ SlotState sst;
-    const int slot = slot0 + blockIdx.x;
+    constexpr int NBI = (Q + kBI - 1) / kBI;
+    static_assert(NBI <= kMaxSplit, "a part for every row block");
+    constexpr int split = SPREAD ? NBI : 1, NIB = SPREAD ? 1 : NBI;
+    const int qd = blockIdx.x >> 3;
+    const int local = SPREAD ? (qd / split) * 8 + (blockIdx.x & 7) : blockIdx.x;
+    const int share = SPREAD ? qd % split : 0;
+    if (SPREAD && local >= slots) return;
+    const int slot = slot0 + local;
     SlotState *st = a.state + slot;
     if (threadIdx.x == 0) sst = *st;
     __syncthreads();
     const int phase = uniform(sst.phase);
     const SlotWorkL<Q, R> w(a.work, slot);
     if (phase == kEmpty) {
+        if (share != 0) return;
         setup_instance<Q, R, kBlock>(a, w, sst);
         if (threadIdx.x == 0) *st = sst;
         return;
@@ -1804,14 +1820,26 @@ __global__ void __launch_bounds__(kBlock) gemm_large_round_kernel(DecimateArgs a
     if (phase != kGemm) return;
     const int par = uniform((sst.it - 1) & 1);
     const int n = a.n;
-    dual_gemm_blocked<Q, R, 0>(lds, red, w.alpha(par), w.beta(par), w.g, n, w.m1, w.m2, nullptr);
+    dual_gemm_blocked<Q, R, 0, NIB>(lds, red, w.alpha(par), w.beta(par), w.g, n, w.m1, w.m2, nullptr,
+                                    share);
     __syncthreads();
-    dual_gemm_blocked<Q, R, 1>(lds, red, w.m1, w.m2, w.beta(par), n, nullptr, w.beta_next(par), w.es);
+    dual_gemm_blocked<Q, R, 1, NIB>(lds, red, w.m1, w.m2, w.beta(par), n, nullptr, w.beta_next(par),
+                                    w.es, share);
     __syncthreads();
-    const double s = dual_gemm_blocked<Q, R, 2>(lds, red, w.m2, w.m1, w.alpha(par), n, nullptr,
-                                                 w.alpha_next(par), w.et);
+    double s = dual_gemm_blocked<Q, R, 2, NIB>(lds, red, w.m2, w.m1, w.alpha(par), n, nullptr,
+                                               w.alpha_next(par), w.et, share);
     if (threadIdx.x == 0) {
+        if constexpr (SPREAD) {
+            __hip_atomic_store(&st->part[share], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __threadfence();
+            if (atomicAdd(&st->arrived, 1u) + 1 < (unsigned)split) return;
+            __threadfence();
+            s = 0.0;
+            for (int k = 0; k < split; ++k)
+                s += __hip_atomic_load(&st->part[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
         SlotState v = sst;
+        v.arrived = 0;
         if (s <= a.accuracy) {
             v.phase = kFinal0;
         } else if (v.it >= a.itermax) {
@@ -1904,7 +1932,7 @@ int padded_q(int n) { return (n + 15) / 16; }
 int decimate_max_q() { return kMaxQ; }
 
 template <int Q, typename R>
-static int launch_round(const DecimateArgs &a, int per_set, int set, bool gj, hipStream_t s) {
+static int launch_round(const DecimateArgs &a, int per_set, int set, bool gj, bool spread, hipStream_t s) {
     if constexpr (std::is_same_v<R, float> ? Q > 5 : Q <= 7) {
         // no FP32 kernels beyond order 80 (the C ABI refuses that case); FP64
         // rounds up to order 112 are mid.hip's
@@ -1925,9 +1953,16 @@ static int launch_round(const DecimateArgs &a, int per_set, int set, bool gj, hi
         if (gj)
             hipLaunchKernelGGL((gj_large_round_kernel<Q, R>), dim3(per_set), dim3(kBlock), gj_lds, s,
                                a, set * per_set);
-        else
-            hipLaunchKernelGGL((gemm_large_round_kernel<Q, R>), dim3(per_set), dim3(kBlock), 0, s, a,
-                               set * per_set);
+        else {
+            constexpr int NBI = (Q + kBI - 1) / kBI;
+            if (spread)
+                hipLaunchKernelGGL((gemm_large_round_kernel<Q, R, true>),
+                                   dim3((per_set + 7) / 8 * 8 * NBI), dim3(kBlock), 0, s, a,
+                                   set * per_set, per_set);
+            else
+                hipLaunchKernelGGL((gemm_large_round_kernel<Q, R, false>), dim3(per_set), dim3(kBlock),
+                                   0, s, a, set * per_set, per_set);
+        }
     }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -1937,10 +1972,11 @@ static int launch_round(const DecimateArgs &a, int per_set, int set, bool gj, hi
         X(21) X(22) X(23) X(24)
 
 template <typename R>
-static int dispatch_round(const DecimateArgs &a, int q, int per_set, int set, bool gj, hipStream_t s) {
+static int dispatch_round(const DecimateArgs &a, int q, int per_set, int set, bool gj, bool spread,
+                          hipStream_t s) {
     switch (q) {
 #define WTSURF_CASE(Q) \
-    case Q: return launch_round<Q, R>(a, per_set, set, gj, s);
+    case Q: return launch_round<Q, R>(a, per_set, set, gj, spread, s);
         WTSURF_FOR_EACH_Q(WTSURF_CASE)
 #undef WTSURF_CASE
         default: return -1;
@@ -1996,9 +2032,9 @@ size_t decimate_slot_bytes(int q, int precision) {
 }
 
 static int launch_phase(const DecimateArgs &a, int q, int precision, int per_set, int set, bool gj,
-                        hipStream_t s) {
-    return precision == 0 ? dispatch_round<double>(a, q, per_set, set, gj, s)
-                          : dispatch_round<float>(a, q, per_set, set, gj, s);
+                        bool spread, hipStream_t s) {
+    return precision == 0 ? dispatch_round<double>(a, q, per_set, set, gj, spread, s)
+                          : dispatch_round<float>(a, q, per_set, set, gj, spread, s);
 }
 
 int decimate_run(const DecimateArgs &a, int q, int precision, int per_set, const RoundCtl &ctl) {
@@ -2014,6 +2050,13 @@ int decimate_run(const DecimateArgs &a, int q, int precision, int per_set, const
     // instances.  Past that bound (with slack) the device has stopped making
     // progress and the run fails instead of launching rounds forever.
     const long slots = (long)NS * per_set;
+    // Beyond order 112 a product or inverse workgroup fills its CU.  While one
+    // set's inverses hold per_set CUs, the other's products have num_cu -
+    // per_set: with fewer than 0.4 num_cu slots a set their row blocks are
+    // spread over the CUs left (150 instances of order 288, 75 a set: 146 ->
+    // 107 ms; one instance 117 -> 53), with more there is nothing to gain and
+    // the operands are read again (300 of order 216 in halves: 96 -> 99 ms).
+    const bool spread = 5 * per_set <= 2 * ctl.num_cu;
     const long per_slot = (a.ninst + slots - 1) / slots + 1;
     const long max_batches = per_slot * (a.itermax + 4) / kRoundsPerBatch + 4;
     if (hipMemsetAsync(a.state, 0, (size_t)slots * sizeof(SlotState), s0) != hipSuccess ||
@@ -2035,8 +2078,8 @@ int decimate_run(const DecimateArgs &a, int q, int precision, int per_set, const
         for (int r = 0; r < kRoundsPerBatch; ++r)
             for (int k = 0; k < NS; ++k) {
                 const bool gj_first = (k & 1) == 0;
-                if (launch_phase(a, q, precision, per_set, k, gj_first, ctl.s[k]) ||
-                    launch_phase(a, q, precision, per_set, k, !gj_first, ctl.s[k]))
+                if (launch_phase(a, q, precision, per_set, k, gj_first, spread, ctl.s[k]) ||
+                    launch_phase(a, q, precision, per_set, k, !gj_first, spread, ctl.s[k]))
                     return -1;
             }
         const int h = (int)(b & 1);

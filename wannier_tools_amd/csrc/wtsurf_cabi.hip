@@ -506,6 +506,7 @@ static int run_decimation(wtsurf_ctx *c, const RunBufs &b, int ninst, int nk, in
     ctl.s[kSlotSets] = c->cnt;
     for (int i = 0; i < kRoundEvents; ++i) ctl.ev[i] = c->drv[i];
     ctl.pinned = c->pinned;
+    ctl.num_cu = c->num_cu;
     const bool mid = use_mid(c, n, precision);
     if (int r = mid ? decimate_mid_run(a, b.plan, static_cast<MidState *>(b.state), c->num_cu, ctl)
                     : decimate_run(a, q, precision, b.per_set, ctl)) {

@@ -8,12 +8,16 @@
 namespace wtsurf {
 
 // Decimation state of one instance slot between rounds (device memory).
+// Workgroups that share one slot's GEMM round beyond order 112 at most.
+constexpr int kMaxSplit = 6;
 struct SlotState {
     int phase;              // empty, inverse next, GEMMs next, final inverse 0..2, done
     int t;                  // instance id
     int it;                 // current iteration (1-based)
     int status;             // bit0 singular solve, bit1 not converged
     double dl, dr;          // traces of the final inverses done so far
+    double part[kMaxSplit]; // sum |alpha'| by share of a split GEMM round
+    unsigned arrived;       // shares of the round that are done
 };
 
 // Arguments of one batched decimation launch (surfgreen_1985 over many
@@ -66,6 +70,7 @@ struct RoundCtl {
     hipStream_t s[kSlotSets + 1];
     hipEvent_t ev[kRoundEvents];
     unsigned *pinned;
+    int num_cu;
 };
 
 int padded_q(int n);        // NP/16 for order n
