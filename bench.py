@@ -60,12 +60,12 @@ if ROOT not in sys.path:
 from wannier_tools_amd import model as M  # noqa: E402
 
 TRAFFIC_JSON = "decimation_fp64_ndim72_512x512.traffic.json"
-DECIMATION_KERNELS = ("gj_round_kernel", "gemm_round_kernel")
+DECIMATION_KERNELS = ("mid_inverse_kernel", "mid_gemm_kernel")
 LARGE_KERNELS = ("gj_large_round_kernel", "gemm_large_round_kernel")
 # per workload: traffic file under profiles/, the stage's kernels, what was run
 TRAFFIC = {
-    "grid72": (TRAFFIC_JSON, DECIMATION_KERNELS, "decimation rounds (gj_round_kernel + "
-               "gemm_round_kernel)", "ndim72 512x512 eta=1e-3 eV"),
+    "grid72": (TRAFFIC_JSON, DECIMATION_KERNELS, "decimation rounds (mid_inverse_kernel + "
+               "mid_gemm_kernel)", "ndim72 512x512 eta=1e-3 eV"),
     "plane288": ("decimation_fp64_ndim288_kplane65.traffic.json", LARGE_KERNELS,
                  "decimation rounds (gj_large_round_kernel + gemm_large_round_kernel)",
                  "ndim288 65x65 k-plane omega=0 eta=5e-4 eV"),
