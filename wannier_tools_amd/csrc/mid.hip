@@ -231,8 +231,8 @@ mid_gemm_kernel(void *work, const MidState *__restrict__ state, int slots, int c
 // Gauss-Jordan inverses, one workgroup each, the matrix in the registers of
 // W waves (3 up to order 80, 7 beyond): lane (a = lane % 8, b = lane / 8) of wave w holds rows a + 8 s
 // (s < KT) of columns 8 (w + W t) + b (t < CL).  Partial pivoting on
-// |re| + |im| over the rows not yet used (the izamax rule of zgesv up to
-// 2^-13 of the value), rows never swapped: step c's pivot row p keeps its
+// |re| + |im| over the rows not yet used (the izamax rule of zgesv, the lowest
+// row on ties), rows never swapped: step c's pivot row p keeps its
 // values unscaled, standing for 1/pivot times itself, takes every later step
 // like any other row and is scaled once at the end; element (row r, column c)
 // is then X^-1[step of r][pivot row of step c].
@@ -293,6 +293,35 @@ __device__ __forceinline__ double group_bcast(double d) {
     return __longlong_as_double(r);
 }
 
+// The pivot of column k by whole values, as the search's key; the sign bit is
+// set where no value is positive.
+template <int KT>
+__device__ __forceinline__ int mid_pivot(const double2 (&x)[KT], int used, int a, int k) {
+    double best = 0.0;
+    int row = a;
+#pragma unroll
+    for (int s = 0; s < KT; ++s) {
+        const double v = fabs(x[s].x) + fabs(x[s].y);
+        if (!(used >> s & 1) && v > best) {
+            best = v;
+            row = a + 8 * s;
+        }
+    }
+#pragma unroll
+    for (int off = 8; off < 64; off *= 2) {
+        const double ob = __shfl_xor(best, off, 64);
+        const int orow = __shfl_xor(row, off, 64);
+        if (ob > best || (ob == best && orow < row)) {
+            best = ob;
+            row = orow;
+        }
+    }
+    best = readlane_f64(best, k);
+    row = __builtin_amdgcn_readlane(row, k);
+    return (__double2hiint(best) & ~127) | (8 * (KT - 1 - (row >> 3)) | (7 - (row & 7))) |
+           (best > 0.0 ? 0 : 1 << 31);
+}
+
 // The panel wave: every panel's elimination.  Lane 8 a + b holds rows a + 8 s
 // of the panel's column b; a step's exchanges stay in the registers (DPP,
 // lane reads and one permute), since its latency is what an inverse's time is
@@ -320,23 +349,34 @@ __device__ __forceinline__ void mid_panels(int n, MidGjShared<KT> &sh) {
             // pivot search: the row (first s, then a, the lower the better)
             // in the low 7 bits of the high word of |re| + |im|, so that one
             // integer maximum finds value and row; used rows count as zero,
-            // and so does NaN
-            int key = 0;
+            // and so does NaN.  Where a second row has the same upper bits
+            // (seldom; all rows of a column without a pivot do), mid_pivot()
+            // looks at whole values.
+            int key = 0, key2 = 0;  // the largest of the lane's rows, the next
 #pragma unroll
             for (int s = 0; s < KT; ++s) {
                 const double v = fmax_nocanon(fabs(x[s].x) + fabs(x[s].y), 0.0);
                 const int free = ~(used << (31 - s) >> 31);
-                key = std::max(key, (__double2hiint(v) & free & ~127) | (8 * (KT - 1 - s)));
+                const int ks = (__double2hiint(v) & free & ~127) | (8 * (KT - 1 - s));
+                key2 = imed3(key, key2, ks);
+                key = std::max(key, ks);
             }
             key |= 7 - a;
+            const int top = key;
             key = std::max(key, __builtin_amdgcn_mov_dpp(key, 0x118, 0xf, 0xf, true));  // row_shr:8
-            const int kh = std::max(std::max(__builtin_amdgcn_readlane(key, 8 + k),
-                                             __builtin_amdgcn_readlane(key, 24 + k)),
-                                    std::max(__builtin_amdgcn_readlane(key, 40 + k),
-                                             __builtin_amdgcn_readlane(key, 56 + k)));
-            // (without a pivot -- the column is zero, or NaN -- the steps go
-            // on with the row the low bits name, and the result is dropped)
-            sing |= kh < 128;
+            int kh = std::max(std::max(__builtin_amdgcn_readlane(key, 8 + k),
+                                       __builtin_amdgcn_readlane(key, 24 + k)),
+                              std::max(__builtin_amdgcn_readlane(key, 40 + k),
+                                       __builtin_amdgcn_readlane(key, 56 + k)));
+            constexpr unsigned long long kCol = 0x0101010101010101ull << k;  // lanes of column k
+            const int other = top == kh ? key2 : top;  // the largest of the lane's rows but the pivot
+            if (__ballot(other >= (kh & ~127)) & kCol) {
+                kh = mid_pivot<KT>(x, used, a, k);
+                // (without a pivot -- the column is zero, or NaN -- the steps
+                // go on with row 0, and the result is dropped)
+                sing |= kh < 0;
+                kh &= 0x7fffffff;
+            }
             const int sp = KT - 1 - ((kh & 127) >> 3), ap = 7 - (kh & 7);
             // the pivot row's entry of this lane's column: bitwise selects (an
             // indexed read would put x in scratch)

@@ -57,11 +57,10 @@ __device__ __forceinline__ double2 cmul_fma(double2 a, double2 b) {
     return make_double2(fma(-a.y, b.y, a.x * b.x), fma(a.y, b.x, a.x * b.y));
 }
 
-// The pivot search's key: the high word of |re| + |im| of a free row (NaN and
-// used rows count as zero) over the row's tag in the bits of mask.
-__device__ __forceinline__ int pivot_key(double re, double im, int free, int mask, int tag) {
+// |re| + |im| of a free row; NaN and used rows count as zero.
+__device__ __forceinline__ double pivot_value(double re, double im, int free) {
     const double v = fmax_nocanon(fabs(re) + fabs(im), 0.0);
-    return (__double2hiint(v) & free & ~mask) | tag;
+    return __hiloint2double(__double2hiint(v) & free, __double2loint(v) & free);
 }
 
 // ---- one instance a wave, orders 9 to 16 -----------------------------------
@@ -123,8 +122,7 @@ __device__ __forceinline__ M16 read_c16(const double2 *m, int i, int q) {
 // x = R(X), pads zero: X^-1 to sh.g in natural order, pads zero (the identity if a
 // pivot column is zero or NaN; returns true then).  Gauss-Jordan with
 // partial pivoting on |re| + |im| over the rows not yet used (the izamax rule
-// of zgesv up to 2^-16 of the value, the lowest row on ties), rows never
-// swapped: step c's pivot row p keeps its values unscaled, standing for
+// of zgesv, the lowest row on ties), rows never swapped: step c's pivot row p keeps its values unscaled, standing for
 // 1/pivot times itself, takes every later step like any other row and is
 // scaled once at the end; element (row r, column c) is then X^-1[step of
 // r][pivot row of step c].  Columns are eliminated in panels of 4, one register of
@@ -151,14 +149,31 @@ __device__ __forceinline__ bool inverse16(M16 &x, int n, Lds16 &sh, int lane) {
             const bool pad = !FULL && KS > 2 && k >= kk;
             const int own = (16 * k + i) << 2;
             double fr = lane_f64(own, yr), fi = lane_f64(own, yi);
-            int key = pivot_key(yr, yi, free, 15, 15 - i);
+            // pivot search: the largest high word, and among several rows that
+            // have it (seldom) the largest low word
+            const double v = pivot_value(yr, yi, free);
+            const int hi = __double2hiint(v);
+            int key = hi;
             key = std::max(key, __builtin_amdgcn_mov_dpp(key, 0x111, 0xf, 0xf, true));  // row_shr:1
             key = std::max(key, __builtin_amdgcn_mov_dpp(key, 0x112, 0xf, 0xf, true));
             key = std::max(key, __builtin_amdgcn_mov_dpp(key, 0x114, 0xf, 0xf, true));
             key = std::max(key, __builtin_amdgcn_mov_dpp(key, 0x118, 0xf, 0xf, true));
             const int kh = __builtin_amdgcn_readlane(key, 16 * k + 15);
-            sing |= !pad && kh < 16;
-            const int p = pad ? 4 * t + k : 15 - (kh & 15);
+            // (in a column without a positive entry all 16 have the high word 0)
+            constexpr int sh0 = 32 * (k / 2), sh1 = 16 * (k % 2);
+            unsigned rows = (unsigned)(__ballot(hi == kh) >> sh0) & (0xffffu << sh1);
+            if (!pad && (rows & (rows - 1))) {
+                const unsigned lo = hi == kh ? (unsigned)__double2loint(v) : 0u;
+                unsigned m = lo;
+                m = std::max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x111, 0xf, 0xf, true));
+                m = std::max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x112, 0xf, 0xf, true));
+                m = std::max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x114, 0xf, 0xf, true));
+                m = std::max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x118, 0xf, 0xf, true));
+                const unsigned ml = (unsigned)__builtin_amdgcn_readlane((int)m, 16 * k + 15);
+                rows = (unsigned)(__ballot(hi == kh && lo == ml) >> sh0) & (0xffffu << sh1);
+                sing |= kh == 0 && ml == 0;
+            }
+            const int p = pad ? 4 * t + k : __builtin_ctz(rows) - sh1;
             const int src = (p | (lane & 48)) << 2;
             const double2 y = make_double2(lane_f64(src, yr), lane_f64(src, yi));
             double2 r = crecip_scaled(make_double2(readlane_f64(yr, 16 * k + p),
@@ -395,6 +410,13 @@ struct M4 {
     double re[KB][KB], im[KB][KB];
 };
 
+// d of the lane that quad_perm CTRL names.
+template <int CTRL>
+__device__ __forceinline__ double quad_f64(double d) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(d), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(d), CTRL, 0xf, 0xf, true));
+}
+
 __device__ __forceinline__ double mfma4(double a, double b, double c) {
     return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
 }
@@ -503,16 +525,38 @@ __device__ __forceinline__ bool inverse4(M4<KB> &x, int n, Lds4<KB> &sh, int lan
             const bool pad = !FULL && k >= kk;
             const int own = (16 * k + (lane & 15)) << 2;
             double2 f[KB];  // the step's column, to every lane of its rows
-            int key = 0;
+            // pivot search: the high word of |re| + |im| over the row's tag;
+            // where a second row of one of the instances has the same upper
+            // bits (seldom), the largest value and the lowest row that has it
+            int key = 0, next = 0;  // the larger of the lane's rows, the other
 #pragma unroll
             for (int I = 0; I < KB; ++I) {
                 f[I] = make_double2(lane_f64(own, x.re[I][t]), lane_f64(own, x.im[I][t]));
-                key = std::max(key, pivot_key(f[I].x, f[I].y, free[I], 15, 15 - 4 * I - i));
+                const int kI = (__double2hiint(pivot_value(f[I].x, f[I].y, free[I])) & ~15) | (15 - 4 * I - i);
+                next = I == 0 ? 0 : std::min(key, kI);
+                key = std::max(key, kI);
             }
-            key = std::max(key, __builtin_amdgcn_mov_dpp(key, 0xB1, 0xf, 0xf, true));  // quad_perm 1,0,3,2
-            key = std::max(key, __builtin_amdgcn_mov_dpp(key, 0x4E, 0xf, 0xf, true));  // quad_perm 2,3,0,1
-            sing |= !pad && key < 16;
-            const int p = pad ? 4 * t + k : 15 - (key & 15);
+            int top = key;
+            top = std::max(top, __builtin_amdgcn_mov_dpp(top, 0xB1, 0xf, 0xf, true));  // quad_perm 1,0,3,2
+            top = std::max(top, __builtin_amdgcn_mov_dpp(top, 0x4E, 0xf, 0xf, true));  // quad_perm 2,3,0,1
+            if (!pad && __ballot((key == top ? next : key) >= (top & ~15))) {
+                double v[KB], best = 0.0;
+#pragma unroll
+                for (int I = 0; I < KB; ++I) {
+                    v[I] = pivot_value(f[I].x, f[I].y, free[I]);
+                    best = fmax_nocanon(best, v[I]);
+                }
+                best = fmax_nocanon(best, quad_f64<0xB1>(best));
+                best = fmax_nocanon(best, quad_f64<0x4E>(best));
+                int tag = 0;
+#pragma unroll
+                for (int I = 0; I < KB; ++I) tag = std::max(tag, v[I] == best ? 15 - 4 * I - i : 0);
+                tag = std::max(tag, __builtin_amdgcn_mov_dpp(tag, 0xB1, 0xf, 0xf, true));
+                tag = std::max(tag, __builtin_amdgcn_mov_dpp(tag, 0x4E, 0xf, 0xf, true));
+                sing |= !(best > 0.0);
+                top = (__double2hiint(best) & ~15) | tag;
+            }
+            const int p = pad ? 4 * t + k : 15 - (top & 15);
             double sr = x.re[0][t], si = x.im[0][t];
             if constexpr (KB == 2)
                 if (p >= 4) {
@@ -534,7 +578,7 @@ __device__ __forceinline__ bool inverse4(M4<KB> &x, int n, Lds4<KB> &sh, int lan
                                               pivot([](double2 z) { return __double2loint(z.x); })),
                              __hiloint2double(pivot([](double2 z) { return __double2hiint(z.y); }),
                                               pivot([](double2 z) { return __double2loint(z.y); }))),
-                (key >> 20) - 1022);
+                (top >> 20) - 1022);
             if (pad) r = make_double2(0.0, 0.0);
             double2 u = cmul_fma(y, r);
             const bool mine = q == k;

@@ -59,6 +59,13 @@ __device__ __forceinline__ double fmax_nocanon(double a, double b) {
     return r;
 }
 
+// Median of three, one instruction.
+__device__ __forceinline__ int imed3(int a, int b, int c) {
+    int r;
+    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
 // Maximum over the 64 lanes of a wave of values whose maximum is >= 0
 // (operands as fmax_nocanon), returned to every lane: DPP row shifts inside
 // each row of 16 lanes, then row broadcasts 15 and 31 carry the partial
@@ -82,26 +89,6 @@ __device__ __forceinline__ double wave_max_f64(double v) {
     WT_DPP_MAX_STEP(0x143, 0xc)  // row_bcast:31
 #undef WT_DPP_MAX_STEP
     return readlane_f64(v, 63);
-}
-
-// Maximum over the 16 lanes of DPP row `row` (lanes 16 row .. 16 row + 15) of
-// values whose maximum there is >= 0, returned to every lane: the four row
-// shifts of wave_max_f64 leave each lane the maximum of its row up to itself,
-// so the row's last lane holds the row's maximum.
-__device__ __forceinline__ double row_max_f64(double v, int row) {
-#define WT_DPP_MAX_STEP(ctrl)                                                         \
-    {                                                                                  \
-        const int hi = __double2hiint(v), lo = __double2loint(v);                      \
-        const int h2 = __builtin_amdgcn_mov_dpp(hi, ctrl, 0xf, 0xf, true);             \
-        const int l2 = __builtin_amdgcn_mov_dpp(lo, ctrl, 0xf, 0xf, true);             \
-        v = fmax_nocanon(v, __hiloint2double(h2, l2));                                 \
-    }
-    WT_DPP_MAX_STEP(0x111)  // row_shr:1
-    WT_DPP_MAX_STEP(0x112)  // row_shr:2
-    WT_DPP_MAX_STEP(0x114)  // row_shr:4
-    WT_DPP_MAX_STEP(0x118)  // row_shr:8
-#undef WT_DPP_MAX_STEP
-    return readlane_f64(v, 16 * row + 15);
 }
 
 // Complex arithmetic on (re, im) pairs of either precision.
