@@ -1369,7 +1369,9 @@ struct GemmLayL {
 // A1 rows and B columns staged through LDS by K-chunks.  kBI kBJ = 24 pairs
 // per block, three per wave.  B is read in every pass, so O1 must not be B.
 // Only NIB row blocks of kBI tiles from ib0 on are formed (and summed); they
-// depend on no other rows of A0 and A1.
+// depend on no other rows of A0 and A1.  In MODE 2 the sum of |O1| is formed row
+// block by row block, so that it does not depend on which workgroup forms
+// which; red: NIB kWaves.
 template <int Q, typename R, int MODE, int NIB>
 __device__ __forceinline__ double dual_gemm_blocked(unsigned char *lds, double *red,
                                                     const typename Prec<R>::C *__restrict__ A0,
@@ -1399,8 +1401,11 @@ __device__ __forceinline__ double dual_gemm_blocked(unsigned char *lds, double *
     // staging: A elements e = tid + u kBlock of a chunk (kk = e / RI, row e % RI),
     // B elements e = tid + u kBlock (kk = e % kChunkL, column e / kChunkL)
 
-    double asum = 0.0;
+    double rsum[NIB];
+#pragma unroll
+    for (int i = 0; i < NIB; ++i) rsum[i] = 0.0;
     for (int blk = 0; blk < NIB * NBJ; ++blk) {
+        double asum = 0.0;
         const int i0 = kBI * (ib0 + blk % NIB), j0 = kBJ * (blk / NIB);
         const int ni = Q - i0 < kBI ? Q - i0 : kBI, nj = Q - j0 < kBJ ? Q - j0 : kBJ;
         int ti[PPW], tj[PPW];
@@ -1488,15 +1493,26 @@ __device__ __forceinline__ double dual_gemm_blocked(unsigned char *lds, double *
         for (int s = 0; s < PPW; ++s)
             if (act[s])
                 store_tile<Q, R, MODE == 2>(i0 + ti[s], j0 + tj[s], lr, lq, pR[s][1], pI[s][1], O1, asum);
+        if (MODE == 2) {
+#pragma unroll
+            for (int i = 0; i < NIB; ++i) rsum[i] += blk % NIB == i ? asum : 0.0;
+        }
     }
     if (MODE == 2) {
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) asum += __shfl_xor(asum, off, 64);
-        if (lane == 0) red[wave] = asum;
+        for (int i = 0; i < NIB; ++i) {
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) rsum[i] += __shfl_xor(rsum[i], off, 64);
+            if (lane == 0) red[i * kWaves + wave] = rsum[i];
+        }
         __syncthreads();
         double tot = 0.0;
+        for (int i = 0; i < NIB; ++i) {
+            double part = 0.0;
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) tot += red[w];
+            for (int w = 0; w < kWaves; ++w) part += red[i * kWaves + w];
+            tot += part;
+        }
         return tot;
     }
     return 0.0;
@@ -1790,13 +1806,14 @@ gemm_round_kernel(DecimateArgs a, int slot0) {
 // row blocks go to one workgroup, or (SPREAD) to one each (on one XCD, whose L2
 // then serves g, alpha and beta to all of them): the rows of all three
 // products depend on the same rows of alpha and beta only.  The last of them to
-// finish adds their parts of sum |alpha'| in order and applies the stop rule.
+// finish adds their parts of sum |alpha'| in order and applies the stop rule;
+// one workgroup alone adds the same parts in the same order.
 // (With the share a run-time number the unspread rounds took 1% longer.)
 template <int Q, typename R, bool SPREAD>
 __global__ void __launch_bounds__(kBlock) gemm_large_round_kernel(DecimateArgs a, int slot0,
                                                                   int slots) {
     __shared__ __align__(16) unsigned char lds[GemmLayL<Q, R>::bytes];
-    __shared__ double red[kWaves];
+    __shared__ double red[kMaxSplit * kWaves];
     __shared__ SlotState sst;
     constexpr int NBI = (Q + kBI - 1) / kBI;
     static_assert(NBI <= kMaxSplit, "a part for every row block");

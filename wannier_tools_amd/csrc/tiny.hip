@@ -380,11 +380,17 @@ tiny16_kernel(DecimateArgs a) {
             write16(d, sh.al, i, q);
             __builtin_amdgcn_sched_barrier(0);
             // stop when sum_ij |alpha'_ij| <= accuracy (:120-122)
+            // (up to order 8 in the order of tiny4_kernel: columns, halves of
+            // the rows, columns, rows)
             double asum = 0.0;
 #pragma unroll
             for (int v = 0; v < 4; ++v) asum += cabs_scaled(d.re[v], d.im[v]);
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) asum += __shfl_xor(asum, off, 64);
+            asum += __shfl_xor(asum, 8, 64);
+            asum += __shfl_xor(asum, 4, 64);
+            asum += __shfl_xor(asum, 32, 64);
+            asum += __shfl_xor(asum, 16, 64);
+            asum += __shfl_xor(asum, 2, 64);
+            asum += __shfl_xor(asum, 1, 64);
             const bool conv = uniform(asum <= a.accuracy);
             if (conv || it >= a.itermax) {
                 if (!conv) status |= 2;
@@ -743,15 +749,19 @@ tiny4_kernel(DecimateArgs a) {
             wave_order();
             write4<KB>(d, sh.al, i, b, q);
             __builtin_amdgcn_sched_barrier(0);
+            // (in the order of tiny16_kernel)
             double asum = 0.0;
 #pragma unroll
-            for (int I = 0; I < KB; ++I)
+            for (int I = 0; I < KB; ++I) {
+                double rsum = 0.0;
 #pragma unroll
-                for (int J = 0; J < KB; ++J) asum += cabs_scaled(d.re[I][J], d.im[I][J]);
-            asum += __shfl_xor(asum, 1, 64);
-            asum += __shfl_xor(asum, 2, 64);
-            asum += __shfl_xor(asum, 16, 64);
+                for (int J = 0; J < KB; ++J) rsum += cabs_scaled(d.re[I][J], d.im[I][J]);
+                asum += rsum;
+            }
             asum += __shfl_xor(asum, 32, 64);
+            asum += __shfl_xor(asum, 16, 64);
+            asum += __shfl_xor(asum, 2, 64);
+            asum += __shfl_xor(asum, 1, 64);
             const bool conv = asum <= a.accuracy;
             if (live && (conv || it >= a.itermax)) {
                 if (!conv) status |= 2;
@@ -793,7 +803,7 @@ int decimate_tiny_run(const DecimateArgs &a, int num_cu, hipStream_t s) {
     // for 80,601 instances of order 16.  Up to one instance a SIMD an instance
     // of order 8 is faster alone in its wave, whose pivots are then uniform
     // (one instance 222 us as one of four, 160 us alone; the same bits, since
-    // the steps and the order of every sum of products are the same).
+    // the steps and the order of every sum are the same).
     const bool full = a.n % 4 == 0, alone = a.n > 8 || a.ninst <= 4L * num_cu;
     auto one = [&](auto kernel) { return launch_tiny(kernel, a, 1, kTinyOcc, num_cu, s); };
     auto four = [&](auto kernel, int occ) { return launch_tiny(kernel, a, 4, occ, num_cu, s); };
