@@ -909,6 +909,21 @@ MidPlan decimate_mid_plan(int ninst, int num_cu) {
     return p;
 }
 
+void decimate_mid_limit(MidPlan &p, int num_cu, size_t most) {
+    const size_t slots = std::max(most, (size_t)2 * num_cu);
+    if ((size_t)p.sets * p.per_set > slots) p.per_set = (int)(slots / p.sets);
+}
+
+bool decimate_mid_halve(MidPlan &p) {
+    if (p.per_set > 1)
+        p.per_set = (p.per_set + 1) / 2;
+    else if (p.sets > 1)
+        p.sets = 1;
+    else
+        return false;
+    return true;
+}
+
 int decimate_mid_run(const DecimateArgs &a, const MidPlan &plan, MidState *state, int num_cu,
                      const RoundCtl &ctl) {
     const int kt = (a.n + 7) / 8;

@@ -31,7 +31,11 @@ struct DevBuf {
         p = nullptr;
         n = 0;
         if (want == 0) return 0;
-        if (hipMalloc(&p, want * sizeof(T)) != hipSuccess) return -1;
+        if (hipMalloc(&p, want * sizeof(T)) != hipSuccess) {
+            (void)hipGetLastError();  // not to be taken for a later launch's
+            p = nullptr;
+            return -1;
+        }
         n = want;
         return 0;
     }
@@ -218,11 +222,20 @@ static bool use_mid(const wtsurf_ctx *c, int n, int precision) {
 static int ensure_work(wtsurf_ctx *c, int n, int precision, int ninst) {
     if (use_mid(c, n, precision)) {
         c->plan = decimate_mid_plan(ninst, c->num_cu);
-        const size_t slots = (size_t)c->plan.sets * c->plan.per_set;
-        const size_t want = slots * decimate_mid_slot_bytes(n);
-        if (want > c->work.n && (c->work.release(), c->work.ensure(want)))
-            return c->fail("out of device memory (decimation workspace)");
-        if (c->state.ensure(2 * slots * sizeof(MidState)) || c->queue.ensure(2))
+        const size_t slot = decimate_mid_slot_bytes(n);
+        auto want = [&] { return (size_t)c->plan.sets * c->plan.per_set * slot; };
+        size_t free = 0, total = 0;
+        if (want() > c->work.n && hipMemGetInfo(&free, &total) == hipSuccess)
+            decimate_mid_limit(c->plan, c->num_cu, (free + c->work.n) / 4 / slot);
+        while (want() > c->work.n) {
+            c->work.release();
+            if (!c->work.ensure(want())) break;
+            // the rounds run with any number of slots
+            if (!decimate_mid_halve(c->plan))
+                return c->fail("out of device memory (decimation workspace)");
+        }
+        if (c->state.ensure(2 * (size_t)c->plan.sets * c->plan.per_set * sizeof(MidState)) ||
+            c->queue.ensure(2))
             return c->fail("out of device memory (slot state)");
         return 0;
     }
@@ -543,10 +556,14 @@ static int launch_decimation(wtsurf_ctx *c, int ninst, int nk, int nomega, const
     // The mixed precision was FP64 but for the last sixth of the iterations;
     // the FP64 rounds now take two thirds of the time those took.
     if (precision == WTSURF_MIXED) precision = WTSURF_FP64;
-    if (int r = ensure_work(c, n, precision, ninst)) return r;
+    // the outputs first: the workspace takes what is left
+    c->spin_ninst = 0;
     if (c->dos_l.ensure(ninst) || c->dos_r.ensure(ninst) || c->dos_b.ensure(ninst) ||
         c->iters.ensure(ninst) || c->status.ensure(ninst))
         return c->fail("out of device memory (outputs)");
+    if (c->spin_mode != WTSURF_SPIN_OFF && c->spin.ensure((size_t)6 * ninst))
+        return c->fail("out of device memory (spin traces)");
+    if (int r = ensure_work(c, n, precision, ninst)) return r;
     RunBufs b;
     b.hk = c->hk.p;
     b.dos_l = c->dos_l.p; b.dos_r = c->dos_r.p; b.dos_b = c->dos_b.p;
@@ -554,12 +571,7 @@ static int launch_decimation(wtsurf_ctx *c, int ninst, int nk, int nomega, const
     b.work = c->work.p; b.state = c->state.p; b.queue = c->queue.p;
     b.per_set = c->per_set;
     b.plan = c->plan;
-    c->spin_ninst = 0;
-    double *spin = nullptr;
-    if (c->spin_mode != WTSURF_SPIN_OFF) {
-        if (c->spin.ensure((size_t)6 * ninst)) return c->fail("out of device memory (spin traces)");
-        spin = c->spin.p;
-    }
+    double *spin = c->spin_mode != WTSURF_SPIN_OFF ? c->spin.p : nullptr;
     if (int r = run_decimation(c, b, ninst, nk, nomega, d_omega, eta, divisor, nullptr, n, nw, d_top,
                                ntop, d_bot, nbot, precision, inst, spin))
         return r;

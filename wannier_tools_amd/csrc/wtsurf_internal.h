@@ -122,6 +122,11 @@ constexpr size_t kMidNoallocSlotBytes = (size_t)922112;  // slot of order 80
 int decimate_mid_max_n();
 size_t decimate_mid_slot_bytes(int n);
 MidPlan decimate_mid_plan(int ninst, int num_cu);
+// The plan cut to `most` slots, but to no fewer than two a CU (one launch of each
+// set then still fills the chip).
+void decimate_mid_limit(MidPlan &p, int num_cu, size_t most);
+// Half as many slots; false if there is only one.
+bool decimate_mid_halve(MidPlan &p);
 // a.work: sets * per_set slots of decimate_mid_slot_bytes(a.n); state: 2 * sets
 // * per_set records.  As decimate_run otherwise (-2: no progress).
 int decimate_mid_run(const DecimateArgs &a, const MidPlan &plan, MidState *state, int num_cu,
