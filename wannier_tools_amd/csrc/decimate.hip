@@ -1603,7 +1603,7 @@ __device__ __forceinline__ int setup_instance(const DecimateArgs &a, const W &w,
     if (tid == 0) st.t = (int)atomicAdd(a.queue, 1u);
     __syncthreads();
     const int t = uniform(st.t);
-    if (t >= a.ninst) {
+    if (queue_empty((unsigned)t, a.ninst)) {
         if (tid == 0) st.phase = kDone;
         __syncthreads();
         return kDone;

@@ -731,7 +731,7 @@ mid_inverse_kernel(DecimateArgs a, const MidState *__restrict__ in, MidState *__
         if (tid == 0) sh.tk = (int)atomicAdd(a.queue, 1u);
         __syncthreads();
         t = uniform(sh.tk);
-        if (t >= a.ninst) {
+        if (queue_empty((unsigned)t, a.ninst)) {
             if (tid == 0) {
                 st.phase = kMidDone;
                 out[slot] = st;
@@ -842,10 +842,10 @@ mid_inverse_kernel(DecimateArgs a, const MidState *__restrict__ in, MidState *__
 }
 
 __global__ void mid_clear_kernel(MidState *state, int nstate, unsigned *queue, int *status, int ninst) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nstate) state[i] = MidState{kMidEmpty, 0, 0, 0, 0, 0};
+    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < (unsigned)nstate) state[i] = MidState{kMidEmpty, 0, 0, 0, 0, 0};
     if (i < 2) queue[i] = 0;
-    if (status && i < ninst) status[i] = 0;
+    if (status && i < (unsigned)ninst) status[i] = 0;
 }
 
 template <int KT>
@@ -936,8 +936,8 @@ int decimate_mid_run(const DecimateArgs &a, const MidPlan &plan, MidState *state
     // which forms m1, m2 of its strip again
     const int csplit = std::max(1, std::min(kt, 4 * num_cu / (per * kt)));
     const int nstate = 2 * NS * per;
-    const int nclear = std::max(std::max(nstate, a.ninst), 2);
-    hipLaunchKernelGGL(mid_clear_kernel, dim3((nclear + 255) / 256), dim3(256), 0, s0, state, nstate,
+    const unsigned nclear = std::max(std::max(nstate, a.ninst), 2);
+    hipLaunchKernelGGL(mid_clear_kernel, dim3((nclear + 255u) / 256u), dim3(256), 0, s0, state, nstate,
                        a.queue, a.status, a.ninst);
     if (hipGetLastError() != hipSuccess || hipEventRecord(start, s0) != hipSuccess) return -1;
     for (int k = 1; k < NS; ++k)

@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(64 * W)
         if (tid == 0) cm.s.t = (int)atomicAdd(a.queue, 1u);
         __syncthreads();
         const int t = uniform(cm.s.t);
-        if (t >= a.ninst) break;
+        if (queue_empty((unsigned)t, a.ninst)) break;
         int ik;
         double2 z;
         instance_of(a, t, ik, z);

@@ -296,7 +296,7 @@ tiny16_kernel(DecimateArgs a) {
     const int n = a.n;
     for (;;) {
         const int t = take(a.queue, 1u);
-        if (t >= a.ninst) break;
+        if (queue_empty((unsigned)t, a.ninst)) break;
         int ik;
         double2 z;
         instance_of(a, t, ik, z);
@@ -653,9 +653,9 @@ tiny4_kernel(DecimateArgs a) {
     const int n = a.n;
     for (;;) {
         const int t0 = take(a.queue, 4u);
-        if (t0 >= a.ninst) break;
+        if (queue_empty((unsigned)t0, a.ninst)) break;
         // the last wave's spare lanes repeat the last instance
-        const int t = std::min(t0 + b, a.ninst - 1);
+        const int t = t0 + std::min(b, a.ninst - 1 - t0);
         int ik;
         double2 z;
         instance_of(a, t, ik, z);

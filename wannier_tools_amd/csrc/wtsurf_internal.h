@@ -7,9 +7,16 @@
 
 namespace wtsurf {
 
-// Decimation state of one instance slot between rounds (device memory).
+// Whether a ticket of the instance queue is past its end.  Tickets go on counting
+// there (every wave or slot takes one before it stops), beyond what an int
+// holds for the largest runs.
+constexpr bool queue_empty(unsigned ticket, int ninst) { return ticket >= (unsigned)ninst; }
+static_assert(queue_empty(0x80000003u, 0x7fffffff) && !queue_empty(0x7ffffffeu, 0x7fffffff),
+              "tickets past 2^31");
+
 // Workgroups that share one slot's GEMM round beyond order 112 at most.
 constexpr int kMaxSplit = 6;
+// Decimation state of one instance slot between rounds (device memory).
 struct SlotState {
     int phase;              // empty, inverse next, GEMMs next, final inverse 0..2, done
     int t;                  // instance id
