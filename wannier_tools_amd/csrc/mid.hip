@@ -597,8 +597,6 @@ __device__ __forceinline__ void mid_traces(const DecimateArgs &a, MidGjShared<KT
         for (int i = 0; i < cnt; ++i) s = s - sh.diag[list ? list[i] - 1 + off : i].x;
         (q == 0 ? a.dos_l : q == 1 ? a.dos_r : a.dos_bulk)[o] = s;
         if (extra && a.status) atomicOr(a.status + o, extra);
-        __threadfence();
-        atomicAdd(a.queue + 1, 1u);
     } else if (tid < 4 && a.spin_mode && q < 2) {
         // surfstat sums GRR's spin traces over the top orbital indices,
         // SurfaceDOSkk over the bottom orbitals of the last layer
@@ -720,13 +718,15 @@ mid_inverse_kernel(DecimateArgs a, const MidState *__restrict__ in, MidState *__
     if (!fin && (ended || st.phase == kMidEmpty)) {
         if (ended && tid == 0) {
             // iterations and status of the finished instance; the final
-            // inverses add their singular bits
+            // inverses of this launch add their singular bits, and the host's
+            // streams wait for whole launches
             int ik0;
             double2 z0;
             instance_of(a, t, ik0, z0);
             const int o = a.inst_k ? t : ik0 + a.nk * (t - ik0 * a.nomega);
             if (a.iters) a.iters[o] = st.it;
             if (a.status && st.status) atomicOr(a.status + o, st.status);
+            atomicAdd(a.queue + 1, 1u);
         }
         if (tid == 0) sh.tk = (int)atomicAdd(a.queue, 1u);
         __syncthreads();
@@ -947,7 +947,7 @@ int decimate_mid_run(const DecimateArgs &a, const MidPlan &plan, MidState *state
     // the device has stopped making progress.
     const long per_slot = (a.ninst + (long)NS * per - 1) / ((long)NS * per) + 1;
     const long max_batches = per_slot * (a.itermax + 2) / kMidRoundsPerBatch + 4;
-    const unsigned want = 3u * (unsigned)a.ninst;
+    const unsigned want = (unsigned)a.ninst;
     // Set k starts with an inverse round; the sets' rounds drift as their
     // launches interleave.  The counter stream copies the finished count to
     // pinned memory after every batch, and the host reads the previous
