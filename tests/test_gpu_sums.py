@@ -94,3 +94,29 @@ def test_ham_of_many_k_points(gpu, n, nk):
     for i in (0, 1, nk // 2, nk - 7 if nk > 7 else 0, nk - 1):
         a, b = gpu.ham_qlayer2qlayer(k[i])
         assert np.array_equal(a, h00[i]) and np.array_equal(b, h01[i])
+
+
+@pytest.mark.gpu
+def test_kpath_jdos_of_many_fields(gpu):
+    """More fields than one launch has workgroups for (2^24 of 256 threads)."""
+    nf = (1 << 24) + 5
+    a = np.random.default_rng(0).uniform(0.1, 1.0, (nf, 3, 1))
+    print("many fields", nf, flush=True)
+    got = gpu.kpath_jdos(a)
+    # shifts 0, 1, 2 of a path of three points
+    want = np.stack([a[:, 0] ** 2 + a[:, 1] ** 2 + a[:, 2] ** 2, a[:, 0] * a[:, 1] + a[:, 1] * a[:, 2],
+                     a[:, 0] * a[:, 2]], axis=1)
+    assert np.all(np.abs(got / want - 1) <= 3 * EPS)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nkx,nky,m1,m2,nfield", [(3, 2100, 2, 2060, 2), (2, 2049, 2, 2049, 1)])
+def test_autocorrelation_of_long_second_axis(gpu, nkx, nky, m1, m2, nfield):
+    """A second modulus beyond the library's row length, which the call then
+    takes as columns."""
+    print("long columns", nkx, nky, m1, m2, flush=True)
+    a = np.random.default_rng(nky).uniform(0.1, 1.0, (nfield, nkx, nky))
+    got = gpu.kplane_autocorrelation(a, m1, m2)
+    want = correlation(a, m1, m2)
+    tol = (nfield * m1 * m2 + nkx * nky / (m1 * m2)) * EPS
+    assert np.abs(got / want - 1).max() <= tol

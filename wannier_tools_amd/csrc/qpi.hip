@@ -293,14 +293,16 @@ __global__ void __launch_bounds__(kCorrBlock) kpath_jdos_kernel(const double *__
         if (iq0 + i < nk) dst[(iq0 + i) * ks] = acc[i];
 }
 
-// out_f(iq, j), element (f, j, ik) as above; thread iq of row (j, f).
+// out_f(iq, j), element (f, j, ik) as above; thread iq of row (j, f) = row0 +
+// blockIdx.y.
 __global__ void __launch_bounds__(kCorrBlock) kpath_jdos_long_kernel(const double *__restrict__ a,
                                                                      int nk, int nomega, size_t fs,
-                                                                     size_t js, size_t ks,
+                                                                     size_t js, size_t ks, int row0,
                                                                      double *__restrict__ out) {
-    const int iq = blockIdx.y * kCorrBlock + threadIdx.x;  // 0-based
+    const int iq = blockIdx.x * kCorrBlock + threadIdx.x;  // 0-based
     if (iq >= nk) return;
-    const size_t row = (blockIdx.x / nomega) * fs + (blockIdx.x % nomega) * js;
+    const int rw = row0 + blockIdx.y;
+    const size_t row = (rw / nomega) * fs + (rw % nomega) * js;
     const double *r = a + row;
     const int h = (nk - 1) / 2;
     const int sft = iq + 1 - h;
@@ -325,9 +327,13 @@ int kpath_jdos_launch(const double *fields, int nk, int nomega, int nfield, bool
             hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
             (void)hipGetLastError();  // the launch reports whether the size is accepted
-        const int per = 8 * kCorrBlock / JT;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)nfield * ((nomega + JT - 1) / JT), (nk + per - 1) / per),
-                           dim3(kCorrBlock), lds, s, fields, nk, nomega, fs, js, ks, out);
+        // (a launch has less than 2^32 threads along x: fields in pieces)
+        const int per = 8 * kCorrBlock / JT, nj = (nomega + JT - 1) / JT;
+        const int step = std::max(1, (1 << 22) / nj);
+        for (int f0 = 0; f0 < nfield; f0 += step)
+            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(step, nfield - f0) * nj, (nk + per - 1) / per),
+                               dim3(kCorrBlock), lds, s, fields + f0 * fs, nk, nomega, fs, js, ks,
+                               out + f0 * fs);
     };
     // as many energies as keep two workgroups of LDS on a CU
     constexpr int kMaxLds = 80 * 1024 / sizeof(double);
@@ -338,9 +344,11 @@ int kpath_jdos_launch(const double *fields, int nk, int nomega, int nfield, bool
     else if (nk <= kMaxLds / 2)
         go(kpath_jdos_kernel<1>, 1);
     else
-        hipLaunchKernelGGL(kpath_jdos_long_kernel,
-                           dim3((unsigned)nfield * nomega, (nk + kCorrBlock - 1) / kCorrBlock),
-                           dim3(kCorrBlock), 0, s, fields, nk, nomega, fs, js, ks, out);
+        for (int r0 = 0; r0 < nfield * nomega; r0 += 65535)
+            hipLaunchKernelGGL(kpath_jdos_long_kernel,
+                               dim3((nk + kCorrBlock - 1) / kCorrBlock,
+                                    (unsigned)std::min(65535, nfield * nomega - r0)),
+                               dim3(kCorrBlock), 0, s, fields, nk, nomega, fs, js, ks, r0, out);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
