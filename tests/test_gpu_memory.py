@@ -62,3 +62,16 @@ def test_rounds_with_little_memory_left(gpu, fill, left):
             assert before - free_memory() < left // 2  # leaves memory to others
     finally:
         ctx.close()
+
+
+def test_qpi_sums_give_large_buffers_back(gpu):
+    """A path whose fields take 0.6 GB on the device, and a plane of 0.5 GB:
+    what the calls keep afterwards is bounded."""
+    rng = np.random.default_rng(3)
+    path, plane = rng.uniform(0.0, 1.0, (1, 21, 1_800_000)), rng.uniform(0.0, 1.0, (1, 2, 16_000_000))
+    gpu.kpath_jdos(path[:, :, :100])
+    before = free_memory()
+    gpu.kpath_jdos(path)
+    assert before - free_memory() <= 300 << 20
+    gpu.kplane_autocorrelation(plane, 2, 2048)
+    assert before - free_memory() <= 300 << 20

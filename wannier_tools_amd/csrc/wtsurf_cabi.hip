@@ -818,6 +818,13 @@ int wtsurf_spin_download(wtsurf_ctx *c, double *spin_l, double *spin_r) {
     return 0;
 }
 
+// The QPI sums' buffer grows on demand and is kept for the next call up to a
+// bound (257 x 257 points and four fields take 8 MB, 512 x 512 on a path 34 MB).
+static void trim_qpi(wtsurf_ctx *c) {
+    constexpr size_t kKeepBytes = (size_t)256 << 20;
+    if (c->qpi.n * sizeof(double) > kKeepBytes) c->qpi.release();
+}
+
 int wtsurf_kplane_autocorrelation(wtsurf_ctx *c, int nkx, int nky, int m1, int m2, int nfield,
                                   const double *fields, double *out) {
     if (!c) return -1;
@@ -827,7 +834,7 @@ int wtsurf_kplane_autocorrelation(wtsurf_ctx *c, int nkx, int nky, int m1, int m
     if (m1 > kplane_corr_max_m()) return c->fail("k-plane too large for the autocorrelation kernel");
     if (int r = use_device(c)) return r;
     const size_t plane = (size_t)nkx * nky;
-    DevBuf<double> &buf = c->qpi;  // grown on demand, kept for the next call
+    DevBuf<double> &buf = c->qpi;
     const size_t corr = kplane_corr_doubles(m1, m2, nfield);
     if (buf.ensure((size_t)nfield * plane + (size_t)nfield * m1 * m2 + corr + plane))
         return c->fail("out of device memory (k-plane autocorrelation)");
@@ -849,6 +856,7 @@ int wtsurf_kplane_autocorrelation(wtsurf_ctx *c, int nkx, int nky, int m1, int m
              (e = hipStreamSynchronize(c->stream)) != hipSuccess)
         rc = c->hipfail(e, "download");
     if (rc) (void)hipStreamSynchronize(c->stream);
+    trim_qpi(c);
     return rc;
 }
 
@@ -872,6 +880,7 @@ static int kpath_jdos(wtsurf_ctx *c, int nk, int nomega, int nfield, bool k_fast
              (e = hipStreamSynchronize(c->stream)) != hipSuccess)
         rc = c->hipfail(e, "download");
     if (rc) (void)hipStreamSynchronize(c->stream);
+    trim_qpi(c);
     return rc;
 }
 
