@@ -75,3 +75,22 @@ def test_qpi_sums_give_large_buffers_back(gpu):
     assert before - free_memory() <= 300 << 20
     gpu.kplane_autocorrelation(plane, 2, 2048)
     assert before - free_memory() <= 300 << 20
+
+
+def test_hamiltonians_with_little_memory_left(gpu, fill):
+    """A list of k points whose H00 and H01 fit the card but not a whole piece of
+    the download beside them: bit for bit as with memory to spare."""
+    n, nk = 96, 500
+    irvec, hr = M.synthetic_model(n, 1, 0.4, M.decay_l2(1.5), seed=96).surface_cell()
+    k = np.random.default_rng(4).uniform(-0.5, 0.5, (nk, 2))
+    gpu.set_model_arrays(n, 1, irvec, hr)
+    want = gpu.ham_qlayer2qlayer(k)
+    ctx = SurfaceGF(0)
+    try:
+        ctx.set_model_arrays(n, 1, irvec, hr)
+        fill(200 << 20)  # 147 MB of H00 and H01, 2 x 64 MiB a piece
+        print("little memory", free_memory(), flush=True)
+        got = ctx.ham_qlayer2qlayer(k)
+    finally:
+        ctx.close()
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])

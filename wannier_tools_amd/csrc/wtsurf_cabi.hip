@@ -437,21 +437,28 @@ int wtsurf_ham_qlayer2qlayer(wtsurf_ctx *c, int nk, const double *kpts, double *
     // the pads come off on the device, and whole arrays go to the caller in
     // pieces of at most 64 MiB
     const size_t nn = (size_t)n * n;
-    const int step = (int)std::min<size_t>(nk, std::max<size_t>(1, ((size_t)64 << 20) / (nn * sizeof(double2))));
-    if (c->hpack.ensure(2 * step * nn)) return c->fail("out of device memory (H00, H01)");
-    for (int ik = 0; ik < nk; ik += step) {
+    int step = (int)std::min<size_t>(nk, std::max<size_t>(1, ((size_t)64 << 20) / (nn * sizeof(double2))));
+    while (c->hpack.ensure(2 * step * nn)) {
+        if (step == 1) return c->fail("out of device memory (H00, H01)");
+        step = (step + 1) / 2;
+    }
+    int rc = 0;
+    hipError_t e = hipSuccess;
+    for (int ik = 0; ik < nk && !rc; ik += step) {
         const int m = std::min(step, nk - ik);
         double2 *p0 = c->hpack.p, *p1 = p0 + m * nn;
         if (unpad_launch(c->hk.p + (size_t)ik * 2 * NP * NP, m, n, NP, p0, p1, c->stream))
-            return c->fail("H00/H01 unpadding launch failed");
-        WT_HIP(c, hipMemcpyAsync(h00 + 2 * ik * nn, p0, m * nn * sizeof(double2),
-                                 hipMemcpyDeviceToHost, c->stream));
-        WT_HIP(c, hipMemcpyAsync(h01 + 2 * ik * nn, p1, m * nn * sizeof(double2),
-                                 hipMemcpyDeviceToHost, c->stream));
+            rc = c->fail("H00/H01 unpadding launch failed");
+        else if ((e = hipMemcpyAsync(h00 + 2 * (size_t)ik * nn, p0, m * nn * sizeof(double2),
+                                     hipMemcpyDeviceToHost, c->stream)) != hipSuccess ||
+                 (e = hipMemcpyAsync(h01 + 2 * (size_t)ik * nn, p1, m * nn * sizeof(double2),
+                                     hipMemcpyDeviceToHost, c->stream)) != hipSuccess)
+            rc = c->hipfail(e, "download");
     }
-    WT_HIP(c, hipStreamSynchronize(c->stream));
+    // (also after an error: no copy into the caller's arrays outlives the call)
+    if ((e = hipStreamSynchronize(c->stream)) != hipSuccess && !rc) rc = c->hipfail(e, "download");
     c->nk = 0;  // hk no longer matches an uploaded grid
-    return 0;
+    return rc;
 }
 
 // Per-instance (k index, omega, eta) device arrays for a batch run, or all null
