@@ -15,7 +15,7 @@ is the Fourier sum plus the batched decimation and traces.
     python bench.py --summarize-counters PMC_DIR KERNEL [KERNEL ...]
 
 Prints one JSON line.  The decimation runs as rounds of two kernels on two
-streams (gj_round_kernel and gemm_round_kernel); the roofline figures refer to
+streams (mid_inverse_kernel and mid_gemm_kernel); the roofline figures refer to
 that whole decimation stage, timed with HIP events on the first stream, which
 waits for the second at the end of the stage.  --summarize-rocprof turns the
 rocprofv3 runs of the same command (kernel trace; FETCH_SIZE and WRITE_SIZE
@@ -390,9 +390,9 @@ def run_grid72(args, SurfaceGF) -> dict:
         return {"max_rel_err_A": float(rel.max()), "median_rel_err_A": float(np.median(rel)),
                 "frac_within_1e-6": float(np.mean(rel <= 1e-6)), "per_file": per_file}
 
-    # FP32 working precision (measurement mode) and the mixed precision (which
-    # runs as FP64): speed and error on A against the FP64 path
-    for prec, peak_ in (("fp32", FP32_MFMA_PEAK_TFLOPS), ("mixed", FP64_MFMA_PEAK_TFLOPS)):
+    # FP32 working precision (measurement mode): speed and error on A against
+    # the FP64 path (the mixed precision runs as FP64 and is not timed again)
+    for prec, peak_ in (("fp32", FP32_MFMA_PEAK_TFLOPS),):
         if args.precision not in ("auto", prec):
             continue
         try:
@@ -404,8 +404,6 @@ def run_grid72(args, SurfaceGF) -> dict:
         res[prec] = {"s_per_step": s_p, "solves_per_s": ninst / s_p, "decimate_ms": dec_p,
                      "steps": aux_steps, **rep, "speedup_vs_fp64": s64 / s_p,
                      "iterations_differing_from_fp64": int(np.count_nonzero(out_p[3] != it64))}
-        if prec == "mixed" and "persistent" in sched_res:
-            res[prec]["speedup_vs_fp64_persistent"] = (sched_res["persistent"]["s_per_step"] / s_p)
         log(f"[bench] {prec}: {ninst / s_p:.1f} solves/s, max rel err {rep['max_rel_err_A']:.2e}")
         if rep["max_rel_err_A"] <= 1e-6 and s_p < best[1]:
             best = (prec, s_p, dec_p, peak_)
@@ -430,7 +428,7 @@ def run_grid72(args, SurfaceGF) -> dict:
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": {"fp64": "c128", "fp32": "c64+c128", "mixed": "c128"}[name],
+        "dtype": {"fp64": "c128", "fp32": "c64+c128"}[name],
         "data": "synthetic",
         "config": {"workload": "surface GF k-path x energy grid, 36-orbital synthetic model, Np=2",
                    "ndim": NDIM, "num_wann": NW, "np": NP_, "nr": int(irvec.shape[0]),
@@ -442,9 +440,7 @@ def run_grid72(args, SurfaceGF) -> dict:
                      "kernel": {"fp64": "decimation stage: mid_inverse_kernel<9> + "
                                          "mid_gemm_kernel<9> rounds on two streams",
                                 "fp32": "decimation stage: gj_round_kernel<5, float> + "
-                                        "gemm_round_kernel<5, float, true> rounds on two streams",
-                                "mixed": "decimation stage: mid_inverse_kernel<9> + "
-                                         "mid_gemm_kernel<9> rounds on two streams"}[name],
+                                        "gemm_round_kernel<5, float, true> rounds on two streams"}[name],
                      "flops_per_launch": flops},
         "paths": res,
     }

@@ -33,10 +33,11 @@ enum {
                          Beyond Ndim 80 it diverges on some instances, so runs with
                          Ndim > 80 fail with an error in this mode. */
     WTSURF_MIXED = 2  /* Within 1e-6 of FP64 on A(k, omega), Ndim <= 80, for callers that
-                         allow it.  Runs as WTSURF_FP64: the FP32 working precision holds
-                         that bound in the last sixth of an instance's iterations at most,
-                         and the kernels that switched there took 1.5 times as long as the
-                         FP64 rounds. */
+                         allow it.  Runs as WTSURF_FP64 on the automatic schedule, whatever
+                         wtsurf_set_schedule says, with the same results: the FP32 working
+                         precision holds that bound in the last sixth of an instance's
+                         iterations at most, and the kernels that switched there took 1.5
+                         times as long as the FP64 rounds. */
 };
 
 /* Per-instance status bits (wtsurf_grid_download / wtsurf_spectral_grid). */

@@ -515,3 +515,23 @@ def test_mixed_precision_low_eta_batch_vs_oracle(gpu, oracle_lib, nw, np_, seed)
             worst = max(worst, abs(mine[t] - one[q][0, 0]) / abs(one[q][0, 0]))
     _say("  max rel err vs oracle:", worst)
     assert worst <= 1e-6
+
+
+@pytest.mark.parametrize("nw,np_", [(4, 2), (24, 1), (36, 2), (40, 2)])
+@pytest.mark.parametrize("schedule", ["rounds", "persistent", "auto"])
+def test_mixed_precision_is_fp64_on_the_automatic_schedule(gpu, nw, np_, schedule):
+    """Whatever schedule is set, a mixed run is the automatic FP64 run."""
+    _say("mixed schedule", nw, np_, schedule)
+    irvec, hr = M.synthetic_model(nw, 1, 0.4, M.decay_l2(1.5), seed=nw).surface_cell()
+    gpu.set_model_arrays(nw, np_, irvec, hr)
+    rng = np.random.default_rng(nw)
+    kp, om = rng.uniform(-0.5, 0.5, (3, 2)), rng.uniform(-1, 1, 5) * M.EV2HARTREE
+    eta = 2e-3 * M.EV2HARTREE
+    want = gpu.spectral_grid(kp, om, eta)
+    gpu.set_schedule(schedule)
+    try:
+        got = gpu.spectral_grid(kp, om, eta, precision="mixed")
+    finally:
+        gpu.set_schedule("auto")
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)

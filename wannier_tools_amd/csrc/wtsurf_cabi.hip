@@ -212,15 +212,15 @@ static int sync_orbitals(wtsurf_ctx *c) {
 
 // FP64 rounds of mid.hip's orders: the schedule asked for is the rounds, or
 // automatic above the small kernel's orders, or has no kernel for the order.
-static bool use_mid(const wtsurf_ctx *c, int n, int precision) {
+static bool use_mid(int schedule, int n, int precision) {
     if (precision != WTSURF_FP64 || n > decimate_mid_max_n()) return false;
-    if (c->schedule == WTSURF_SCHEDULE_PERSISTENT && padded_q(n) <= decimate_persistent_max_q())
+    if (schedule == WTSURF_SCHEDULE_PERSISTENT && padded_q(n) <= decimate_persistent_max_q())
         return false;
-    return c->schedule == WTSURF_SCHEDULE_ROUNDS || n > decimate_small_max_n();
+    return schedule == WTSURF_SCHEDULE_ROUNDS || n > decimate_small_max_n();
 }
 
-static int ensure_work(wtsurf_ctx *c, int n, int precision, int ninst) {
-    if (use_mid(c, n, precision)) {
+static int ensure_work(wtsurf_ctx *c, int schedule, int n, int precision, int ninst) {
+    if (use_mid(schedule, n, precision)) {
         c->plan = decimate_mid_plan(ninst, c->num_cu);
         const size_t slot = decimate_mid_slot_bytes(n);
         auto want = [&] { return (size_t)c->plan.sets * c->plan.per_set * slot; };
@@ -479,6 +479,7 @@ struct RunBufs {
     unsigned *queue = nullptr;
     int per_set = 0;
     MidPlan plan;
+    int schedule = WTSURF_SCHEDULE_AUTO;
 };
 
 // Enqueue the rounds of one decimation run on the context streams.
@@ -501,7 +502,7 @@ static int run_decimation(wtsurf_ctx *c, const RunBufs &b, int ninst, int nk, in
     }
     const int q = padded_q(n);
     if (precision == WTSURF_FP64 && n <= decimate_small_max_n() &&
-        (c->schedule == WTSURF_SCHEDULE_SMALL || c->schedule == WTSURF_SCHEDULE_AUTO)) {
+        (b.schedule == WTSURF_SCHEDULE_SMALL || b.schedule == WTSURF_SCHEDULE_AUTO)) {
         if (decimate_small_run(a, c->num_cu, c->stream)) {
             const hipError_t e = hipGetLastError();
             return e != hipSuccess ? c->hipfail(e, "small-order decimation")
@@ -509,7 +510,7 @@ static int run_decimation(wtsurf_ctx *c, const RunBufs &b, int ninst, int nk, in
         }
         return 0;
     }
-    if (c->schedule == WTSURF_SCHEDULE_PERSISTENT && q <= decimate_persistent_max_q()) {
+    if (b.schedule == WTSURF_SCHEDULE_PERSISTENT && q <= decimate_persistent_max_q()) {
         // one workgroup per CU (at most one per instance), slots 0.. of the workspace
         const int nblocks = std::min(c->num_cu, ninst);
         if (nblocks > kSlotSets * b.per_set) return c->fail("decimation workspace too small");
@@ -527,7 +528,7 @@ static int run_decimation(wtsurf_ctx *c, const RunBufs &b, int ninst, int nk, in
     for (int i = 0; i < kRoundEvents; ++i) ctl.ev[i] = c->drv[i];
     ctl.pinned = c->pinned;
     ctl.num_cu = c->num_cu;
-    const bool mid = use_mid(c, n, precision);
+    const bool mid = use_mid(b.schedule, n, precision);
     if (int r = mid ? decimate_mid_run(a, b.plan, static_cast<MidState *>(b.state), c->num_cu, ctl)
                     : decimate_run(a, q, precision, b.per_set, ctl)) {
         for (auto s : c->aux) (void)hipStreamSynchronize(s);  // rounds already queued there
@@ -545,6 +546,7 @@ static int check_order(wtsurf_ctx *c, int n, int precision) {
     if (precision == WTSURF_FP32 && q > 5)
         return c->fail("WTSURF_FP32 is limited to Ndim <= 80: beyond that the doubling "
                        "recursion in FP32 diverges on some instances (use WTSURF_FP64)");
+    // (the orders that mode has always taken)
     if (precision == WTSURF_MIXED && q > decimate_persistent_max_q())
         return c->fail("WTSURF_MIXED is built for Ndim <= 80 (use WTSURF_FP64)");
     return 0;
@@ -560,8 +562,11 @@ static int launch_decimation(wtsurf_ctx *c, int ninst, int nk, int nomega, const
                              const int *d_bot, int nbot, int precision,
                              InstanceLists inst = InstanceLists()) {
     if (int r = check_order(c, n, precision)) return r;
-    // The mixed precision was FP64 but for the last sixth of the iterations;
-    // the FP64 rounds now take two thirds of the time those took.
+    // The mixed precision was FP64 but for the last sixth of the iterations, on
+    // kernels of its own whatever the schedule; FP64 on the automatic schedule
+    // takes two thirds of the time those took.
+    RunBufs b;
+    b.schedule = precision == WTSURF_MIXED ? (int)WTSURF_SCHEDULE_AUTO : c->schedule;
     if (precision == WTSURF_MIXED) precision = WTSURF_FP64;
     // the outputs first: the workspace takes what is left
     c->spin_ninst = 0;
@@ -570,8 +575,7 @@ static int launch_decimation(wtsurf_ctx *c, int ninst, int nk, int nomega, const
         return c->fail("out of device memory (outputs)");
     if (c->spin_mode != WTSURF_SPIN_OFF && c->spin.ensure((size_t)6 * ninst))
         return c->fail("out of device memory (spin traces)");
-    if (int r = ensure_work(c, n, precision, ninst)) return r;
-    RunBufs b;
+    if (int r = ensure_work(c, b.schedule, n, precision, ninst)) return r;
     b.hk = c->hk.p;
     b.dos_l = c->dos_l.p; b.dos_r = c->dos_r.p; b.dos_b = c->dos_b.p;
     b.iters = c->iters.p; b.status = c->status.p;
@@ -611,11 +615,12 @@ int wtsurf_surfgreen_1985(wtsurf_ctx *c, int n, double omega, double eta, const 
     // buffers of their own (grown on demand, kept for the next call), so that
     // the grid's H00/H01, energies and outputs stay as the last grid run left them
     if (c->hk1.ensure(pad.size()) || c->one_d.ensure(4) || c->one_i.ensure(3) ||
-        c->gfull.ensure((size_t)3 * n * n) || ensure_work(c, n, WTSURF_FP64, 1))
+        c->gfull.ensure((size_t)3 * n * n) || ensure_work(c, c->schedule, n, WTSURF_FP64, 1))
         return c->fail("out of device memory");
     WT_HIP(c, hipMemcpy(c->hk1.p, pad.data(), pad.size() * sizeof(double2), hipMemcpyHostToDevice));
     WT_HIP(c, hipMemcpy(c->one_d.p + 3, &omega, sizeof(double), hipMemcpyHostToDevice));
     RunBufs b;
+    b.schedule = c->schedule;
     b.hk = c->hk1.p;
     b.dos_l = c->one_d.p; b.dos_r = c->one_d.p + 1; b.dos_b = c->one_d.p + 2;
     b.iters = c->one_i.p; b.status = c->one_i.p + 1;
@@ -667,6 +672,7 @@ int wtsurf_surfgreen_1985_noalloc(wtsurf_ctx *c, int n, double omega, double eta
     WT_HIP(c, hipMemcpy2DAsync(hk + (size_t)NP * NP, prow, d_h01, row, row, n,
                                hipMemcpyDeviceToDevice, c->stream));
     RunBufs b;
+    b.schedule = c->schedule;
     b.hk = hk;
     b.dos_l = outs; b.dos_r = outs + 1; b.dos_b = outs + 2;
     b.iters = iouts; b.status = iouts + 1;
