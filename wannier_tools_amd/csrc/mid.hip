@@ -843,7 +843,7 @@ mid_inverse_kernel(DecimateArgs a, const MidState *__restrict__ in, MidState *__
 
 __global__ void mid_clear_kernel(MidState *state, int nstate, unsigned *queue, int *status, int ninst) {
     const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < (unsigned)nstate) state[i] = MidState{kMidEmpty, 0, 0, 0, 0, 0};
+    if (i < (unsigned)nstate) state[i] = MidState{kMidEmpty, 0, 0, 0, 0};
     if (i < 2) queue[i] = 0;
     if (status && i < (unsigned)ninst) status[i] = 0;
 }

@@ -23,7 +23,11 @@
 
 namespace wtsurf {
 
-template <int NP, int W>
+namespace {
+
+constexpr int NP = 32;  // order of the padded matrices (as H00 and H01 are stored)
+constexpr int W = 8;    // waves per instance
+
 struct SmallCfg {
     static constexpr int NT = 64 * W;
     static constexpr int NC = NT / NP;
@@ -31,12 +35,10 @@ struct SmallCfg {
     static constexpr int GPW = 64 / NP;  // column groups per wave
     static constexpr int LD = NP + 1;
     static constexpr int MAT = NP * LD;
-    static constexpr int NPG = NP < 16 ? 16 : NP;  // order of the H00/H01 arrays (16-padded)
-    static_assert(64 % NP == 0 && NT % NP == 0 && NP % NC == 0, "layout must tile the workgroup");
+    static_assert(64 % NP == 0 && W > 1 && NT % NP == 0 && NP % NC == 0, "layout must tile the workgroup");
 };
 
 // Pivot exchange of the Gauss-Jordan steps, double-buffered by step parity.
-template <int NP>
 struct SmallPivot {
     double2 mcol[2][NP];  // multipliers X[i][c] / pivot (0 for the pivot row)
     double2 rr[2];        // 1 / pivot
@@ -44,12 +46,11 @@ struct SmallPivot {
     int sing[2];          // zero pivot column
 };
 
-template <int NP, int W>
 struct SmallLay {
-    using Cfg = SmallCfg<NP, W>;
+    using Cfg = SmallCfg;
     // alpha, beta, g (then m1), m2
     static constexpr size_t mats = (size_t)4 * Cfg::MAT * sizeof(double2);
-    static constexpr size_t bytes = mats + sizeof(SmallPivot<NP>);
+    static constexpr size_t bytes = mats + sizeof(SmallPivot);
 };
 
 // Element (i, j) of a natural-order LDS matrix.
@@ -73,10 +74,9 @@ struct SmallG {
 // the pivot lane of its column group.  Returns true on an exactly zero pivot
 // column; G then holds the identity, as the reference's inv hands back
 // (src/inverse.f90:44-55).
-template <int NP, int W, int E = SmallCfg<NP, W>::EPL>
-__device__ __forceinline__ bool small_gj(double2 (&x)[E], int n,
-                                         SmallPivot<NP> &sh, double2 *G) {
-    using Cfg = SmallCfg<NP, W>;
+__device__ __forceinline__ bool small_gj(double2 (&x)[SmallCfg::EPL], int n,
+                                         SmallPivot &sh, double2 *G) {
+    using Cfg = SmallCfg;
     constexpr int NC = Cfg::NC, EPL = Cfg::EPL, GPW = Cfg::GPW, LD = Cfg::LD;
     const int tid = threadIdx.x;
     const int wave = uniform(tid >> 6), lane = tid & 63;
@@ -167,12 +167,12 @@ __device__ __forceinline__ bool small_gj(double2 (&x)[E], int n,
 }
 
 // P0 = A0 B and P1 = A1 B over K = n, the thread's own elements of each.
-template <int NP, int W, int E = SmallCfg<NP, W>::EPL>
 __device__ __forceinline__ void small_dual(const double2 *__restrict__ A0,
                                            const double2 *__restrict__ A1,
                                            const double2 *__restrict__ B, int n,
-                                           double2 (&p0)[E], double2 (&p1)[E]) {
-    using Cfg = SmallCfg<NP, W>;
+                                           double2 (&p0)[SmallCfg::EPL],
+                                           double2 (&p1)[SmallCfg::EPL]) {
+    using Cfg = SmallCfg;
     constexpr int NC = Cfg::NC, EPL = Cfg::EPL, LD = Cfg::LD;
     const int tid = threadIdx.x;
     const int i = tid % NP, jc = tid / NP;
@@ -192,42 +192,36 @@ __device__ __forceinline__ void small_dual(const double2 *__restrict__ A0,
     }
 }
 
-template <int NP, int W, int E = SmallCfg<NP, W>::EPL>
-__device__ __forceinline__ void small_store(double2 *M, const double2 (&p)[E]) {
-    using Cfg = SmallCfg<NP, W>;
+__device__ __forceinline__ void small_store(double2 *M, const double2 (&p)[SmallCfg::EPL]) {
+    using Cfg = SmallCfg;
     const int tid = threadIdx.x;
     const int i = tid % NP, jc = tid / NP;
 #pragma unroll
     for (int u = 0; u < Cfg::EPL; ++u) M[i + (jc + Cfg::NC * u) * Cfg::LD] = p[u];
 }
 
-// Workgroups per CU: as many as the LDS holds (with the static part), at most
-// 24 (order 8: more would cap the registers below what its loops hold); and
-// the waves per SIMD that gives, which caps the registers of the kernel
-// (512 / waves per SIMD).
-template <int NP, int W>
+// Workgroups per CU: as many as the LDS holds (with the static part); and the
+// waves per SIMD that gives, which caps the registers of the kernel (512 /
+// waves per SIMD).
 constexpr int small_per_cu() {
-    constexpr size_t per = SmallLay<NP, W>::bytes + sizeof(Common<(NP + 15) / 16>) + W * sizeof(double) + 256;
-    constexpr size_t k = (size_t)160 * 1024 / per;
-    return k < 1 ? 1 : k > 24 ? 24 : (int)k;
+    constexpr size_t per = SmallLay::bytes + sizeof(Common<NP / 16>) + W * sizeof(double) + 256;
+    return (int)((size_t)160 * 1024 / per);
 }
-template <int NP, int W>
 constexpr int small_waves_per_simd() {
-    constexpr int w = (small_per_cu<NP, W>() * W + 3) / 4;
+    constexpr int w = (small_per_cu() * W + 3) / 4;
     return w > 8 ? 8 : w;
 }
 
-template <int NP, int W>
 __global__ void __launch_bounds__(64 * W)
-    __attribute__((amdgpu_waves_per_eu(small_waves_per_simd<NP, W>())))
+    __attribute__((amdgpu_waves_per_eu(small_waves_per_simd())))
     small_kernel(DecimateArgs a) {
-    using Cfg = SmallCfg<NP, W>;
-    constexpr int NC = Cfg::NC, EPL = Cfg::EPL, LD = Cfg::LD, MAT = Cfg::MAT, NPG = Cfg::NPG;
-    constexpr int QC = (NP + 15) / 16;
+    using Cfg = SmallCfg;
+    constexpr int NC = Cfg::NC, EPL = Cfg::EPL, LD = Cfg::LD, MAT = Cfg::MAT;
+    constexpr int QC = NP / 16;
     extern __shared__ __align__(16) unsigned char lds[];
     double2 *AL = reinterpret_cast<double2 *>(lds);
     double2 *BE = AL + MAT, *GM = BE + MAT, *M2 = GM + MAT;
-    SmallPivot<NP> &sh = *reinterpret_cast<SmallPivot<NP> *>(lds + SmallLay<NP, W>::mats);
+    SmallPivot &sh = *reinterpret_cast<SmallPivot *>(lds + SmallLay::mats);
     __shared__ Common<QC> cm;
     __shared__ double red[W];
     const int tid = threadIdx.x;
@@ -242,8 +236,8 @@ __global__ void __launch_bounds__(64 * W)
         int ik;
         double2 z;
         instance_of(a, t, ik, z);
-        const double2 *H00 = a.hk + (size_t)ik * 2 * NPG * NPG;
-        const double2 *H01 = H00 + NPG * NPG;
+        const double2 *H00 = a.hk + (size_t)ik * 2 * NP * NP;
+        const double2 *H01 = H00 + NP * NP;
         // eps_s = eps_t = H00, alpha = H01, beta = H01^dagger (src/surfgreen.f90:74-78)
         double2 es[EPL], et[EPL], h0[EPL];
 #pragma unroll
@@ -251,9 +245,9 @@ __global__ void __launch_bounds__(64 * W)
             const int j = jc + NC * u;
             double2 h = make_double2(0.0, 0.0), al = h, be = h;
             if (i < n && j < n) {
-                h = H00[i + j * NPG];
-                al = H01[i + j * NPG];
-                const double2 ht = H01[j + i * NPG];
+                h = H00[i + j * NP];
+                al = H01[i + j * NP];
+                const double2 ht = H01[j + i * NP];
                 be = make_double2(ht.x, -ht.y);
             }
             es[u] = et[u] = h0[u] = h;
@@ -273,22 +267,22 @@ __global__ void __launch_bounds__(64 * W)
                 if (i >= n || j >= n) x[u] = make_double2(0.0, 0.0);
             }
             __syncthreads();  // the set-up or the last products are in LDS, GM is free
-            if (small_gj<NP, W>(x, n, sh, GM)) status |= 1;
+            if (small_gj(x, n, sh, GM)) status |= 1;
             double2 p0[EPL], p1[EPL];
             // m1 = alpha g, m2 = beta g (:92-95)
-            small_dual<NP, W>(AL, BE, GM, n, p0, p1);
+            small_dual(AL, BE, GM, n, p0, p1);
             __syncthreads();  // every read of g done: m1 takes its place
-            small_store<NP, W>(GM, p0);
-            small_store<NP, W>(M2, p1);
+            small_store(GM, p0);
+            small_store(M2, p1);
             __syncthreads();
             // eps_s += m1 beta, beta' = m2 beta (:98-102, 116-117)
-            small_dual<NP, W>(GM, M2, BE, n, p0, p1);
+            small_dual(GM, M2, BE, n, p0, p1);
 #pragma unroll
             for (int u = 0; u < EPL; ++u) es[u] = cadd(es[u], p0[u]);
             __syncthreads();
-            small_store<NP, W>(BE, p1);
+            small_store(BE, p1);
             // eps_t += m2 alpha, alpha' = m1 alpha (:107-114)
-            small_dual<NP, W>(M2, GM, AL, n, p0, p1);
+            small_dual(M2, GM, AL, n, p0, p1);
             double asum = 0.0;
 #pragma unroll
             for (int u = 0; u < EPL; ++u) {
@@ -296,7 +290,7 @@ __global__ void __launch_bounds__(64 * W)
                 asum += hypot(p1[u].x, p1[u].y);
             }
             __syncthreads();
-            small_store<NP, W>(AL, p1);
+            small_store(AL, p1);
             // stop when sum_ij |alpha'_ij| <= accuracy (:120-122)
 #pragma unroll
             for (int off = 32; off >= 1; off >>= 1) asum += __shfl_xor(asum, off, 64);
@@ -328,7 +322,7 @@ __global__ void __launch_bounds__(64 * W)
                 if (i >= n || j >= n) x[u] = make_double2(0.0, 0.0);
             }
             __syncthreads();  // the previous final's traces are done with GM
-            if (small_gj<NP, W>(x, n, sh, GM)) status |= 1;
+            if (small_gj(x, n, sh, GM)) status |= 1;
             for (int e = tid; e < n; e += Cfg::NT) cm.diag[e] = GM[e + e * LD];
             if (a.gfull) {
                 double2 *full = a.gfull + ((size_t)t * 3 + q) * n * n;
@@ -345,25 +339,26 @@ __global__ void __launch_bounds__(64 * W)
     }
 }
 
-template <int NP, int W>
 static int launch_small(const DecimateArgs &a, int num_cu, hipStream_t s) {
-    constexpr size_t lds = SmallLay<NP, W>::bytes;
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&small_kernel<NP, W>),
+    constexpr size_t lds = SmallLay::bytes;
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&small_kernel),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         (void)hipGetLastError();  // the launch reports whether the size is accepted
-    const long want = (long)num_cu * small_per_cu<NP, W>();
+    const long want = (long)num_cu * small_per_cu();
     const int nblocks = (int)std::max<long>(1, std::min<long>(want, a.ninst));
-    hipLaunchKernelGGL((small_kernel<NP, W>), dim3(nblocks), dim3(64 * W), lds, s, a);
+    hipLaunchKernelGGL(small_kernel, dim3(nblocks), dim3(64 * W), lds, s, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int decimate_small_max_n() { return 32; }
+}  // namespace
+
+int decimate_small_max_n() { return NP; }
 
 int decimate_small_run(const DecimateArgs &a, int num_cu, hipStream_t s) {
     if (a.n < 1 || a.n > decimate_small_max_n() || num_cu < 1) return -1;
     if (hipMemsetAsync(a.queue, 0, 2 * sizeof(unsigned), s) != hipSuccess) return -1;
     if (a.n <= decimate_tiny_max_n()) return decimate_tiny_run(a, num_cu, s);
-    return launch_small<32, 8>(a, num_cu, s);
+    return launch_small(a, num_cu, s);
 }
 
 }  // namespace wtsurf

@@ -120,7 +120,6 @@ struct MidState {
     int it;      // current iteration (1-based)
     int status;  // bit0 singular solve, bit1 not converged
     int buf;     // which of the slot's two states the iteration reads
-    int pad;
 };
 struct MidPlan {
     int sets = 1, per_set = 1;  // slot sets (one stream each) and slots per set
