@@ -120,3 +120,23 @@ def test_autocorrelation_of_long_second_axis(gpu, nkx, nky, m1, m2, nfield):
     want = correlation(a, m1, m2)
     tol = (nfield * m1 * m2 + nkx * nky / (m1 * m2)) * EPS
     assert np.abs(got / want - 1).max() <= tol
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nkx,nky,m1,m2,nfield", [(1, 40, 1, 39, 1), (2, 300, 2, 300, 1), (33, 40, 33, 31, 2),
+                                                  (40, 33, 31, 33, 2), (200, 5, 129, 5, 3)])
+def test_autocorrelation_of_narrow_rows(gpu, nkx, nky, m1, m2, nfield):
+    """Narrow planes through the library in both orders of the axes, and the
+    Python call, which takes the longer axis as rows."""
+    print("narrow rows", nkx, nky, m1, m2, nfield, flush=True)
+    a = np.random.default_rng(nkx + nky).uniform(0.1, 1.0, (nfield, nkx, nky))
+    want = correlation(a, m1, m2)
+    p = lambda v: v.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+    lib, ctx = gpu.lib, gpu.ctx
+    b = np.ascontiguousarray(a.transpose(0, 2, 1))
+    c1, c2 = np.zeros((nkx, nky)), np.zeros((nky, nkx))
+    assert lib.wtsurf_kplane_autocorrelation(ctx, nky, nkx, m2, m1, nfield, p(a), p(c1)) == 0
+    assert lib.wtsurf_kplane_autocorrelation(ctx, nkx, nky, m1, m2, nfield, p(b), p(c2)) == 0
+    tol = (nfield * m1 * m2 + nkx * nky / (m1 * m2)) * EPS
+    for got in (gpu.kplane_autocorrelation(a, m1, m2), c1, c2.T):
+        assert np.abs(got / want - 1).max() <= tol

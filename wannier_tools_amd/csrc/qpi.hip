@@ -81,7 +81,7 @@ __host__ __device__ __forceinline__ constexpr int row_length(int len) { return (
 template <int R2>
 __global__ void __launch_bounds__(kCorrBlock) correlate_kernel(
     const double *__restrict__ a, const double *__restrict__ e, int nkx, int nky, int m1, int m2,
-    int nfield, int TP, int len, double *__restrict__ part) {
+    int nfield, int TP, int JN, int len, double *__restrict__ part) {
     extern __shared__ __align__(16) double lds[];
     const int G = kCorrBlock / TP;
     const int ld = row_length(len);
@@ -90,6 +90,7 @@ __global__ void __launch_bounds__(kCorrBlock) correlate_kernel(
     double *ar = lds + (size_t)G * le;  // [G + R2 - 1][ld]
     const int tid = threadIdx.x;
     const int tp = tid % TP, g = tid / TP;
+    const int sj = tid % JN, srow = 4 * (tid / JN), sstep = 4 * (kCorrBlock / JN);
     const int p20 = R2 * blockIdx.x;
     const int chunks = (m2 + G - 1) / G;  // per field
     const long total = (long)nfield * chunks;
@@ -105,10 +106,11 @@ __global__ void __launch_bounds__(kCorrBlock) correlate_kernel(
         const double *ef = e + ((size_t)f * m2 + c20) * m1;
         const double *af = a + (size_t)f * nkx * nky;
         __syncthreads();  // the previous rows are no longer read
-        // (four loads in flight a thread)
+        // (JN threads along a row, the others on other rows; four loads in
+        // flight a thread)
         const int p2 = (c20 + p20) % m2, rows = ng + R2 - 1;
-        for (int j = tid; j < m1; j += kCorrBlock) {
-            for (int row = 0; row < rows; row += 4) {
+        for (int j = sj; j < m1; j += JN) {
+            for (int row = srow; row < rows; row += sstep) {
                 double v[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
@@ -121,7 +123,7 @@ __global__ void __launch_bounds__(kCorrBlock) correlate_kernel(
                     for (int x = j; x < len; x += m1)  // around the torus
                         ar[std::min(row + u, rows - 1) * ld + skew(x)] = v[u];
             }
-            for (int row = 0; row < ng; row += 4) {
+            for (int row = srow; row < ng; row += sstep) {
                 double v[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) v[u] = ef[(size_t)std::min(row + u, ng - 1) * m1 + j];
@@ -353,17 +355,21 @@ int kpath_jdos_launch(const double *fields, int nk, int nomega, int nfield, bool
 }
 
 // Launch shape of correlate_kernel: threads along p1 (a power of two, so that
-// the groups of threads tile the workgroup), the LDS length of a row of a, R2
-// as large as two workgroups of LDS a CU allow, and slices for about four
-// workgroups a CU.
+// the groups of threads tile the workgroup), threads along a row when rows are
+// staged (a power of two: all of them stage narrow rows too, at m1 = 1, m2 =
+// 2000 0.2 ms for 7.1 with one thread to a row's element), the LDS length of a row of
+// a, R2 as large as two workgroups of LDS a CU allow, and slices for about
+// four workgroups a CU.
 struct CorrPlan {
-    int tp, len, r2, slices;
+    int tp, jn, len, r2, slices;
     size_t lds;
 };
 static CorrPlan corr_plan(int m1, int m2, int nfield) {
     CorrPlan p{};
     p.tp = 8;
     while (8 * p.tp < m1) p.tp *= 2;
+    p.jn = 1;
+    while (p.jn < m1 && p.jn < kCorrBlock) p.jn *= 2;
     p.len = m1 + 8 * p.tp + 8;
     const int G = kCorrBlock / p.tp;
     for (p.r2 = 4;; p.r2 /= 2) {
@@ -396,8 +402,8 @@ int kplane_corr_launch(const KplaneCorrArgs &k, hipStream_t s) {
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds) != hipSuccess)
             (void)hipGetLastError();  // the launch reports whether the size is accepted
         hipLaunchKernelGGL(kernel, dim3((k.m2 + p.r2 - 1) / p.r2, p.slices), dim3(kCorrBlock), p.lds,
-                           s, k.fields, k.folded, k.nkx, k.nky, k.m1, k.m2, k.nfield, p.tp, p.len,
-                           k.corr);
+                           s, k.fields, k.folded, k.nkx, k.nky, k.m1, k.m2, k.nfield, p.tp, p.jn,
+                           p.len, k.corr);
     };
     if (p.r2 == 4)
         go(correlate_kernel<4>);

@@ -304,9 +304,11 @@ class SurfaceGF:
         if f.ndim == 2:
             f = f[None]
         nfield, nkx, nky = f.shape
-        if max(m1, m2) <= 2048:
+        if max(m1, m2) <= 2048 and m2 >= min(m1, 32):
             # the sum is the same with the axes exchanged, and so is its result:
-            # no transposes (the library limits the length of its rows)
+            # no transposes (the library limits the length of its rows, and is
+            # at its best with long ones: 1025 x 3 points 1.0 ms as rows of 2,
+            # 0.1 as rows of 1024)
             buf = np.ascontiguousarray(f)
             out = np.empty((nkx, nky), dtype=np.float64)
             self._check(self.lib.wtsurf_kplane_autocorrelation(
