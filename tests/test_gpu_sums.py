@@ -123,6 +123,33 @@ def test_autocorrelation_of_long_second_axis(gpu, nkx, nky, m1, m2, nfield):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nk,nom,nfield", [(1, 1, 1), (15, 256, 1), (40, 256, 1), (40, 257, 1), (41, 3, 2),
+                                           (5121, 2, 1), (5121, 11, 1), (10240, 2, 1), (10240, 7, 1), (10241, 3, 2),
+                                           (10241, 7, 1)])
+def test_kpath_jdos_where_the_kernel_changes(gpu, nk, nom, nfield):
+    """Short paths of few rows, one workgroup's LDS, and paths beyond it in both
+    orders: against 80-bit sums of positive terms, within nk eps."""
+    print("jdos kernels", nk, nom, nfield, flush=True)
+    a = np.random.default_rng(nk + nom).uniform(0.1, 1.0, (nfield, nk, nom))
+    h = (nk - 1) // 2
+    x = a[:, :2 * h + 1].astype(np.longdouble)
+    got = gpu.kpath_jdos(a)
+    src = np.ascontiguousarray(a.transpose(0, 2, 1))
+    got_k = np.zeros_like(src)
+    p = lambda v: v.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+    assert gpu.lib.wtsurf_kpath_jdos(gpu.ctx, nk, nom, nfield, p(src), p(got_k)) == 0
+    assert np.array_equal(got, got_k.transpose(0, 2, 1))
+    for iq in sorted({0, 1 % nk, h, min(h + 1, nk - 1), max(nk - 2, 0), nk - 1, nk // 3}):
+        s = iq + 1 - h
+        lo, hi = max(0, -s), min(2 * h, 2 * h - s)
+        if hi < lo:
+            assert np.all(got[:, iq] == 0)
+            continue
+        want = (x[:, lo:hi + 1] * x[:, lo + s:hi + s + 1]).sum(axis=1)
+        assert np.all(np.abs(got[:, iq] / want - 1) <= nk * EPS)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("nkx,nky,m1,m2,nfield", [(1, 40, 1, 39, 1), (2, 300, 2, 300, 1), (33, 40, 33, 31, 2),
                                                   (40, 33, 31, 33, 2), (200, 5, 129, 5, 3)])
 def test_autocorrelation_of_narrow_rows(gpu, nkx, nky, m1, m2, nfield):

@@ -37,8 +37,10 @@
 // consecutive shifts, sliding an 8-wide window over the path: two LDS reads for
 // eight multiply-adds (one thread per sum from global memory: 388 us at 512 x
 // 512 and four fields, 50 us staged), and the same kernel reads either order of the arrays
-// (k or energy fastest), so that no caller transposes.  Paths too long for LDS take kpath_jdos_long_kernel,
-// one thread per (iq, j, field) from global memory.
+// (k or energy fastest), so that no caller transposes.  Paths too long for LDS,
+// and the smallest calls, take kpath_jdos_long_kernel, one thread per (iq, j,
+// field) from global memory; long paths with the energy fastest are exchanged
+// on the device first, for its loads' sake.
 #include <algorithm>
 
 #include "wtsurf_device.h"
@@ -251,10 +253,10 @@ __global__ void __launch_bounds__(kCorrBlock) kpath_jdos_kernel(const double *__
     int lo[8], hi[8], first = nk, last = -1, from = 0, to = nk;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const int sft = iq0 + i + 1 - h;
+        // (past the last shift: that one again, not stored)
+        const int sft = min(iq0 + i, nk - 1) + 1 - h;
         lo[i] = sft < 0 ? -sft : 0;                 // 0-based first ik
         hi[i] = sft > 0 ? 2 * h - sft : 2 * h;      // 0-based last ik
-        if (iq0 + i >= nk) hi[i] = lo[i] - 1;       // no such shift
         acc[i] = 0.0;
         if (hi[i] >= lo[i]) {
             first = min(first, lo[i]);
@@ -269,13 +271,13 @@ __global__ void __launch_bounds__(kCorrBlock) kpath_jdos_kernel(const double *__
         const double x = r[ik * LD];
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-            if (ik >= lo[i] && ik <= hi[i]) acc[i] = fma(x, r[(ik + s0 + i) * LD], acc[i]);
+            if (ik >= lo[i] && ik <= hi[i]) acc[i] = fma(x, r[min(ik + s0 + i, nk - 1) * LD], acc[i]);
     };
     int ik = first;
     for (; ik < from && ik <= last; ++ik) edge(ik);
     if (ik + 7 <= to) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) w[i] = r[(ik + s0 + i) * LD];
+        for (int i = 0; i < 8; ++i) w[i] = r[min(ik + s0 + i, nk - 1) * LD];
         for (; ik + 7 <= to; ik += 8) {
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
@@ -295,8 +297,8 @@ __global__ void __launch_bounds__(kCorrBlock) kpath_jdos_kernel(const double *__
         if (iq0 + i < nk) dst[(iq0 + i) * ks] = acc[i];
 }
 
-// out_f(iq, j), element (f, j, ik) as above; thread iq of row (j, f) = row0 +
-// blockIdx.y.
+// out_f(iq, j) from global memory, element (f, j, ik) as above; thread iq of row
+// (j, f) = row0 + blockIdx.y.
 __global__ void __launch_bounds__(kCorrBlock) kpath_jdos_long_kernel(const double *__restrict__ a,
                                                                      int nk, int nomega, size_t fs,
                                                                      size_t js, size_t ks, int row0,
@@ -315,9 +317,27 @@ __global__ void __launch_bounds__(kCorrBlock) kpath_jdos_long_kernel(const doubl
     out[row + iq * ks] = s;
 }
 
+// dst [nfield][cols][rows] = src [nfield][rows][cols]
+__global__ void __launch_bounds__(kCorrBlock) transpose_kernel(const double *__restrict__ src, int rows,
+                                                               int cols, long total,
+                                                               double *__restrict__ dst) {
+    const long plane = (long)rows * cols;
+    for (long e = blockIdx.x * (long)kCorrBlock + threadIdx.x; e < total; e += (long)gridDim.x * kCorrBlock) {
+        const long f = e / plane, r = e - f * plane;
+        dst[e] = src[f * plane + (r % rows) * cols + r / rows];
+    }
+}
+
 }  // namespace
 
 int kplane_corr_max_m() { return kKplaneMaxM; }
+
+int transpose_launch(const double *src, int rows, int cols, int nfield, double *dst, hipStream_t s) {
+    const long total = (long)rows * cols * nfield;
+    const unsigned blocks = (unsigned)std::min<long>((total + kCorrBlock - 1) / kCorrBlock, 1 << 16);
+    hipLaunchKernelGGL(transpose_kernel, dim3(blocks), dim3(kCorrBlock), 0, s, src, rows, cols, total, dst);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
+}
 
 int kpath_jdos_launch(const double *fields, int nk, int nomega, int nfield, bool k_fastest,
                       double *out, hipStream_t s) {
@@ -337,20 +357,22 @@ int kpath_jdos_launch(const double *fields, int nk, int nomega, int nfield, bool
                                dim3(kCorrBlock), lds, s, fields + f0 * fs, nk, nomega, fs, js, ks,
                                out + f0 * fs);
     };
-    // as many energies as keep two workgroups of LDS on a CU
+    // as many energies as keep two workgroups of LDS on a CU, or at last one;
+    // the smallest calls are a launch's latency, and staging only adds to it
+    // (21 points and energies: 36 us from global memory, 40 staged)
     constexpr int kMaxLds = 80 * 1024 / sizeof(double);
-    if (nk <= kMaxLds / 17)
-        go(kpath_jdos_kernel<16>, 16);
-    else if (nk <= kMaxLds / 5)
-        go(kpath_jdos_kernel<4>, 4);
-    else if (nk <= kMaxLds / 2)
-        go(kpath_jdos_kernel<1>, 1);
-    else
+    if (nk > kJdosStagedMaxNk || (nk <= 40 && nfield * nomega <= 256)) {
         for (int r0 = 0; r0 < nfield * nomega; r0 += 65535)
             hipLaunchKernelGGL(kpath_jdos_long_kernel,
                                dim3((nk + kCorrBlock - 1) / kCorrBlock,
                                     (unsigned)std::min(65535, nfield * nomega - r0)),
                                dim3(kCorrBlock), 0, s, fields, nk, nomega, fs, js, ks, r0, out);
+    } else if (nk <= kMaxLds / 17)
+        go(kpath_jdos_kernel<16>, 16);
+    else if (nk <= kMaxLds / 5)
+        go(kpath_jdos_kernel<4>, 4);
+    else
+        go(kpath_jdos_kernel<1>, 1);
     return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

@@ -883,12 +883,17 @@ static int kpath_jdos(wtsurf_ctx *c, int nk, int nomega, int nfield, bool k_fast
     if (buf.ensure(2 * n)) return c->fail("out of device memory (k-path jdos)");
     int rc = 0;
     hipError_t e;
-    if ((e = hipMemcpyAsync(buf.p, fields, n * sizeof(double), hipMemcpyHostToDevice, c->stream)) !=
+    // a long path with the energy fastest: the two halves take turns
+    const bool turn = !k_fastest && nk > kJdosStagedMaxNk;
+    double *in = turn ? buf.p + n : buf.p, *res = turn ? buf.p : buf.p + n;
+    if ((e = hipMemcpyAsync(in, fields, n * sizeof(double), hipMemcpyHostToDevice, c->stream)) !=
         hipSuccess)
         rc = c->hipfail(e, "upload");
-    else if (kpath_jdos_launch(buf.p, nk, nomega, nfield, k_fastest, buf.p + n, c->stream))
+    else if ((turn && transpose_launch(in, nk, nomega, nfield, buf.p, c->stream)) ||
+             kpath_jdos_launch(buf.p, nk, nomega, nfield, k_fastest || turn, buf.p + n, c->stream) ||
+             (turn && transpose_launch(buf.p + n, nomega, nk, nfield, res, c->stream)))
         rc = c->fail("k-path jdos launch failed");
-    else if ((e = hipMemcpyAsync(out, buf.p + n, n * sizeof(double), hipMemcpyDeviceToHost,
+    else if ((e = hipMemcpyAsync(out, res, n * sizeof(double), hipMemcpyDeviceToHost,
                                  c->stream)) != hipSuccess ||
              (e = hipStreamSynchronize(c->stream)) != hipSuccess)
         rc = c->hipfail(e, "download");

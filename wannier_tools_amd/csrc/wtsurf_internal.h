@@ -168,6 +168,12 @@ struct KplaneCorrArgs {
 int kplane_corr_max_m();
 size_t kplane_corr_doubles(int m1, int m2, int nfield);
 int kplane_corr_launch(const KplaneCorrArgs &k, hipStream_t s);
+// dst [nfield][cols][rows] = src [nfield][rows][cols], device buffers.
+int transpose_launch(const double *src, int rows, int cols, int nfield, double *dst, hipStream_t s);
+// Longest path that kpath_jdos_launch stages in LDS (160 KB, two doubles a
+// point): 9000 points, 50 rows 4.1 ms from global memory, 1.3 staged; 5121
+// points, four rows 0.47 and 0.50.
+constexpr int kJdosStagedMaxNk = 160 * 1024 / 16;
 // k-path joint density of states (src/surfstat.f90:891-907); device buffers
 // [nfield][nomega][nk] (k_fastest) or [nfield][nk][nomega].
 int kpath_jdos_launch(const double *fields, int nk, int nomega, int nfield, bool k_fastest,
