@@ -39,6 +39,27 @@ __device__ __forceinline__ double lane_f64(int src, double d) {
                             __builtin_amdgcn_ds_bpermute(src, __double2loint(d)));
 }
 
+// d of the lane that the DPP control names.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double d) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(d), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(d), CTRL, 0xf, 0xf, true));
+}
+
+// The sum over lanes l, l ^ 32, then ^ 16, ^ 2, ^ 1, in every lane of them.  (A swap
+// of a value with itself leaves the one half, or the even rows, in the first
+// result and the other in the second.)
+__device__ __forceinline__ double quad_rows_sum(double d) {
+    auto a = __builtin_amdgcn_permlane32_swap(__double2hiint(d), __double2hiint(d), false, false);
+    auto b = __builtin_amdgcn_permlane32_swap(__double2loint(d), __double2loint(d), false, false);
+    d = __hiloint2double(a[0], b[0]) + __hiloint2double(a[1], b[1]);
+    a = __builtin_amdgcn_permlane16_swap(__double2hiint(d), __double2hiint(d), false, false);
+    b = __builtin_amdgcn_permlane16_swap(__double2loint(d), __double2loint(d), false, false);
+    d = __hiloint2double(a[0], b[0]) + __hiloint2double(a[1], b[1]);
+    d += dpp_f64<0x4E>(d);     // quad_perm 2,3,0,1
+    return d + dpp_f64<0xB1>(d);  // quad_perm 1,0,3,2
+}
+
 // The next k tickets of the queue, the first of them to every lane.  The lane
 // number is hidden and the barrier keeps the branch where it is: a compiler
 // that knows which lanes come from the lane 0 branch at the loop's end sends
@@ -69,7 +90,8 @@ struct M16 {
     v4d re, im;
 };
 
-// R(A B) from C(B) and R(A), K = 4 KS.
+// R(A B) from C(B) and R(A), K = 4 KS.  Columns from 4 KS on depend on such
+// columns of B alone, and nothing reads them: they may hold anything.
 template <int KS>
 __device__ __forceinline__ M16 mul16(const M16 &c, const M16 &r) {
     using P = Prec<double>;
@@ -92,9 +114,10 @@ struct Lds16 {
     double2 al[16 * kLd16], be[16 * kLd16];
 };
 
+template <int KS>
 __device__ __forceinline__ void write16(const M16 &r, double2 *m, int i, int q) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) m[(4 * t + q) * kLd16 + i] = make_double2(r.re[t], r.im[t]);
+    for (int t = 0; t < KS; ++t) m[(4 * t + q) * kLd16 + i] = make_double2(r.re[t], r.im[t]);
 }
 template <int KS>
 __device__ __forceinline__ M16 read_r16(const double2 *m, int i, int q) {
@@ -119,34 +142,35 @@ __device__ __forceinline__ M16 read_c16(const double2 *m, int i, int q) {
     return c;
 }
 
-// x = R(X), pads zero: X^-1 to sh.g in natural order, pads zero (the identity if a
-// pivot column is zero or NaN; returns true then).  Gauss-Jordan with
+// x = R(X), the identity (KS <= 2: zero) from row and column n to 4 KS: X^-1 to
+// sh.g in natural order, the identity from there on (the identity of order n if a pivot column is zero or NaN;
+// returns true then).  Gauss-Jordan with
 // partial pivoting on |re| + |im| over the rows not yet used (the izamax rule
 // of zgesv, the lowest row on ties), rows never swapped: step c's pivot row p keeps its values unscaled, standing for
 // 1/pivot times itself, takes every later step like any other row and is
 // scaled once at the end; element (row r, column c) is then X^-1[step of
-// r][pivot row of step c].  Columns are eliminated in panels of 4, one register of
+// r][pivot row of step c].  Rows and columns from n on hold the identity, whose
+// steps change nothing, or (KS <= 2: the time of one instance, and what the
+// registers of larger orders do not allow) zero, whose steps are left out.
+// Columns are eliminated in panels of 4, one register of
 // every lane, and the panel is applied to the rest as X += M T by four MFMA,
 // M the panel's columns (with the distance from 1 where a pivot row meets
 // its own column) and T its pivot rows.
-template <int KS, bool FULL>
+template <int KS>
 __device__ __forceinline__ bool inverse16(M16 &x, int n, Lds16 &sh, int lane) {
     const int i = lane & 15, q = lane >> 4;
-    int free = i < n ? -1 : 0;
-    int srow = i < n ? 1 << 20 : i;  // step at which row i was the pivot (not yet)
+    int free = i < 4 * KS ? -1 : 0;
+    constexpr bool kSkip = KS <= 2;
+    int srow = i < (kSkip ? n : 4 * KS) ? 1 << 20 : i;  // step at which row i was the pivot (not yet)
     double2 myr = make_double2(1.0, 0.0);
     int prow[4] = {q, 4 + q, 8 + q, 12 + q};  // pivot row of the own columns' steps
     int sing = 0;
     auto panel = [&](auto tc) {
         constexpr int t = tc;
-        const int kk = FULL ? 4 : std::min(4, n - 4 * t);
         double yr = x.re[t], yi = x.im[t];
         auto step = [&](auto kc) {
             constexpr int k = kc;
-            // a column beyond n: no step, or (what the registers of larger
-            // orders allow) one that changes nothing
-            if (!FULL && KS <= 2 && k >= kk) return;
-            const bool pad = !FULL && KS > 2 && k >= kk;
+            if (kSkip && 4 * t + k >= n) return;
             const int own = (16 * k + i) << 2;
             double fr = lane_f64(own, yr), fi = lane_f64(own, yi);
             // pivot search: the largest high word, and among several rows that
@@ -162,7 +186,7 @@ __device__ __forceinline__ bool inverse16(M16 &x, int n, Lds16 &sh, int lane) {
             // (in a column without a positive entry all 16 have the high word 0)
             constexpr int sh0 = 32 * (k / 2), sh1 = 16 * (k % 2);
             unsigned rows = (unsigned)(__ballot(hi == kh) >> sh0) & (0xffffu << sh1);
-            if (!pad && (rows & (rows - 1))) {
+            if (rows & (rows - 1)) {
                 const unsigned lo = hi == kh ? (unsigned)__double2loint(v) : 0u;
                 unsigned m = lo;
                 m = std::max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x111, 0xf, 0xf, true));
@@ -171,15 +195,14 @@ __device__ __forceinline__ bool inverse16(M16 &x, int n, Lds16 &sh, int lane) {
                 m = std::max(m, (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x118, 0xf, 0xf, true));
                 const unsigned ml = (unsigned)__builtin_amdgcn_readlane((int)m, 16 * k + 15);
                 rows = (unsigned)(__ballot(hi == kh && lo == ml) >> sh0) & (0xffffu << sh1);
-                sing |= kh == 0 && ml == 0;
+                sing |= kh == 0 && ml == 0 && 4 * t + k < n;
             }
-            const int p = pad ? 4 * t + k : __builtin_ctz(rows) - sh1;
+            const int p = __builtin_ctz(rows) - sh1;
             const int src = (p | (lane & 48)) << 2;
             const double2 y = make_double2(lane_f64(src, yr), lane_f64(src, yi));
             double2 r = crecip_scaled(make_double2(readlane_f64(yr, 16 * k + p),
                                                    readlane_f64(yi, 16 * k + p)),
                                       (kh >> 20) - 1022);
-            if (pad) r = make_double2(0.0, 0.0);
             double2 u = cmul_fma(y, r);
             if (q == k) {
                 u = r;
@@ -197,15 +220,15 @@ __device__ __forceinline__ bool inverse16(M16 &x, int n, Lds16 &sh, int lane) {
         };
         each_of(std::make_integer_sequence<int, 4>(), step);
         const int k = srow - 4 * t;
-        if (k >= 0 && k < kk && i < n) {
+        if (k >= 0 && k < 4) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
+            for (int v = 0; v < KS; ++v)
                 if (v != t) sh.g[20 * k + 4 * v + q] = make_double2(x.re[v], x.im[v]);
         }
         wave_order();
         double2 a = sh.g[20 * q + i];
         wave_order();
-        if (q >= kk || (i >> 2) == t) a = make_double2(0.0, 0.0);
+        if ((i >> 2) == t) a = make_double2(0.0, 0.0);
         x.re[t] = yr;
         x.im[t] = yi;
         using P = Prec<double>;
@@ -213,11 +236,11 @@ __device__ __forceinline__ bool inverse16(M16 &x, int n, Lds16 &sh, int lane) {
         x.im = P::mfma(a.x, yi, x.im);
         x.re = mfma_neg(a.y, yi, x.re);
         x.im = P::mfma(a.y, yr, x.im);
-        if (prow[t] == i && q < kk) x.re[t] += 1.0;
+        if (prow[t] == i) x.re[t] += 1.0;
     };
     each_of(std::make_integer_sequence<int, KS>(), panel);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < KS; ++t) {
         const double2 e = cmul_fma(make_double2(x.re[t], x.im[t]), myr);
         const int c = 4 * t + q;
         if (sing)
@@ -288,7 +311,7 @@ __device__ __forceinline__ void tiny_traces(const DecimateArgs &a, int f, int o,
 // Waves per SIMD: the loops hold about 160 registers, one 4 x 4 tile 80.
 constexpr int kTinyOcc = 3, kTinyOcc1 = 6;
 
-template <int KS, bool FULL>
+template <int KS>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kTinyOcc)))
 tiny16_kernel(DecimateArgs a) {
     __shared__ Lds16 sh;
@@ -302,9 +325,9 @@ tiny16_kernel(DecimateArgs a) {
         instance_of(a, t, ik, z);
         const double2 *H00 = a.hk + (size_t)ik * 512, *H01 = H00 + 256;
         // eps_s = eps_t = H00, alpha = H01, beta = H01^dagger (src/surfgreen.f90:74-78)
-        M16 es, et;
+        M16 es{{0, 0, 0, 0}, {0, 0, 0, 0}}, et;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
+        for (int v = 0; v < KS; ++v) {
             const int c = 4 * v + q;
             const double2 h = H00[i + 16 * c], s = H01[c + 16 * i];
             es.re[v] = h.x;
@@ -322,9 +345,9 @@ tiny16_kernel(DecimateArgs a) {
             // in registers through the loop)
             const int lane = opaque_tid(), i = lane & 15, q = lane >> 4;
             // g = (z - eps_i)^-1, eps_i = eps_s + eps_t - H00 (src/surfgreen.f90:88-89)
-            M16 x;
+            M16 x{{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
+            for (int v = 0; v < KS; ++v) {
                 const double2 h = H00[i + 16 * (4 * v + q)];
                 double ex = (es.re[v] + et.re[v]) - h.x, ey = (es.im[v] + et.im[v]) - h.y;
                 if (f == 0) {
@@ -334,11 +357,11 @@ tiny16_kernel(DecimateArgs a) {
                     ex = et.re[v];
                     ey = et.im[v];
                 }
-                const bool in = (FULL && KS == 4) || (i < n && 4 * v + q < n), dg = i == 4 * v + q;
-                x.re[v] = in ? (dg ? z.x : 0.0) - ex : 0.0;
+                const bool in = i < n && 4 * v + q < n, dg = i == 4 * v + q;
+                x.re[v] = in ? (dg ? z.x : 0.0) - ex : dg && KS > 2 ? 1.0 : 0.0;
                 x.im[v] = in ? (dg ? z.y : 0.0) - ey : 0.0;
             }
-            if (inverse16<KS, FULL>(x, n, sh, lane)) status |= 1;
+            if (inverse16<KS>(x, n, sh, lane)) status |= 1;
             if (f >= 0) {
                 bool up = false;
                 const int pr = a.spin_mode && i < n ? spin_partner(i, a.nw, up) : -1;
@@ -367,7 +390,7 @@ tiny16_kernel(DecimateArgs a) {
             __builtin_amdgcn_sched_barrier(0);
             d = mul16<KS>(c, m2);
             wave_order();
-            write16(d, sh.be, i, q);
+            write16<KS>(d, sh.be, i, q);
             __builtin_amdgcn_sched_barrier(0);
             // eps_t += m2 alpha, alpha' = m1 alpha (:107-114)
             c = read_c16<KS>(sh.al, i, q);
@@ -377,20 +400,17 @@ tiny16_kernel(DecimateArgs a) {
             __builtin_amdgcn_sched_barrier(0);
             d = mul16<KS>(c, m1);
             wave_order();
-            write16(d, sh.al, i, q);
+            write16<KS>(d, sh.al, i, q);
             __builtin_amdgcn_sched_barrier(0);
             // stop when sum_ij |alpha'_ij| <= accuracy (:120-122)
             // (up to order 8 in the order of tiny4_kernel: columns, halves of
             // the rows, columns, rows)
             double asum = 0.0;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) asum += cabs_scaled(d.re[v], d.im[v]);
-            asum += __shfl_xor(asum, 8, 64);
-            asum += __shfl_xor(asum, 4, 64);
-            asum += __shfl_xor(asum, 32, 64);
-            asum += __shfl_xor(asum, 16, 64);
-            asum += __shfl_xor(asum, 2, 64);
-            asum += __shfl_xor(asum, 1, 64);
+            for (int v = 0; v < KS; ++v) asum += cabs_scaled(d.re[v], d.im[v]);
+            asum += dpp_f64<0x128>(asum);  // row_ror:8
+            asum += dpp_f64<0x124>(asum);  // row_ror:4
+            asum = quad_rows_sum(asum);
             const bool conv = uniform(asum <= a.accuracy);
             if (conv || it >= a.itermax) {
                 if (!conv) status |= 2;
@@ -415,13 +435,6 @@ template <int KB>
 struct M4 {
     double re[KB][KB], im[KB][KB];
 };
-
-// d of the lane that quad_perm CTRL names.
-template <int CTRL>
-__device__ __forceinline__ double quad_f64(double d) {
-    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(d), CTRL, 0xf, 0xf, true),
-                            __builtin_amdgcn_mov_dpp(__double2loint(d), CTRL, 0xf, 0xf, true));
-}
 
 __device__ __forceinline__ double mfma4(double a, double b, double c) {
     return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
@@ -510,25 +523,23 @@ __device__ __forceinline__ void write4(const M4<KB> &r, double2 *m, int i, int b
 
 // As inverse16, for the four instances at once; the lanes of a singular one
 // return true.
-template <int KB, bool FULL>
+template <int KB>
 __device__ __forceinline__ bool inverse4(M4<KB> &x, int n, Lds4<KB> &sh, int lane) {
     const int i = lane & 3, b = (lane >> 2) & 3, q = lane >> 4;
     int free[KB], srow[KB], prow[KB];
     double2 myr[KB];
 #pragma unroll
     for (int I = 0; I < KB; ++I) {
-        free[I] = 4 * I + i < n ? -1 : 0;
-        srow[I] = 4 * I + i < n ? 1 << 20 : 4 * I + i;
+        free[I] = -1;
+        srow[I] = 1 << 20;
         prow[I] = 4 * I + q;
         myr[I] = make_double2(1.0, 0.0);
     }
     int sing = 0;
     auto panel = [&](auto tc) {
         constexpr int t = tc;
-        const int kk = FULL ? 4 : std::min(4, n - 4 * t);
         auto step = [&](auto kc) {
             constexpr int k = kc;
-            const bool pad = !FULL && k >= kk;
             const int own = (16 * k + (lane & 15)) << 2;
             double2 f[KB];  // the step's column, to every lane of its rows
             // pivot search: the high word of |re| + |im| over the row's tag;
@@ -545,24 +556,24 @@ __device__ __forceinline__ bool inverse4(M4<KB> &x, int n, Lds4<KB> &sh, int lan
             int top = key;
             top = std::max(top, __builtin_amdgcn_mov_dpp(top, 0xB1, 0xf, 0xf, true));  // quad_perm 1,0,3,2
             top = std::max(top, __builtin_amdgcn_mov_dpp(top, 0x4E, 0xf, 0xf, true));  // quad_perm 2,3,0,1
-            if (!pad && __ballot((key == top ? next : key) >= (top & ~15))) {
+            if (__ballot((key == top ? next : key) >= (top & ~15))) {
                 double v[KB], best = 0.0;
 #pragma unroll
                 for (int I = 0; I < KB; ++I) {
                     v[I] = pivot_value(f[I].x, f[I].y, free[I]);
                     best = fmax_nocanon(best, v[I]);
                 }
-                best = fmax_nocanon(best, quad_f64<0xB1>(best));
-                best = fmax_nocanon(best, quad_f64<0x4E>(best));
+                best = fmax_nocanon(best, dpp_f64<0xB1>(best));
+                best = fmax_nocanon(best, dpp_f64<0x4E>(best));
                 int tag = 0;
 #pragma unroll
                 for (int I = 0; I < KB; ++I) tag = std::max(tag, v[I] == best ? 15 - 4 * I - i : 0);
                 tag = std::max(tag, __builtin_amdgcn_mov_dpp(tag, 0xB1, 0xf, 0xf, true));
                 tag = std::max(tag, __builtin_amdgcn_mov_dpp(tag, 0x4E, 0xf, 0xf, true));
-                sing |= !(best > 0.0);
+                sing |= !(best > 0.0) && 4 * t + k < n;
                 top = (__double2hiint(best) & ~15) | tag;
             }
-            const int p = pad ? 4 * t + k : 15 - (top & 15);
+            const int p = 15 - (top & 15);
             double sr = x.re[0][t], si = x.im[0][t];
             if constexpr (KB == 2)
                 if (p >= 4) {
@@ -585,7 +596,6 @@ __device__ __forceinline__ bool inverse4(M4<KB> &x, int n, Lds4<KB> &sh, int lan
                              __hiloint2double(pivot([](double2 z) { return __double2hiint(z.y); }),
                                               pivot([](double2 z) { return __double2loint(z.y); }))),
                 (top >> 20) - 1022);
-            if (pad) r = make_double2(0.0, 0.0);
             double2 u = cmul_fma(y, r);
             const bool mine = q == k;
             if (mine) {
@@ -611,13 +621,12 @@ __device__ __forceinline__ bool inverse4(M4<KB> &x, int n, Lds4<KB> &sh, int lan
 #pragma unroll
             for (int I = 0; I < KB; ++I) {
                 const int k = srow[I] - 4 * t;
-                if (k >= 0 && k < kk && 4 * I + i < n)
+                if (k >= 0 && k < 4)
                     sh.g[16 * k + 4 * b + q] = make_double2(x.re[I][v], x.im[I][v]);
             }
             wave_order();
             double2 a = sh.g[lane];
             wave_order();
-            if (q >= kk) a = make_double2(0.0, 0.0);
 #pragma unroll
             for (int I = 0; I < KB; ++I) {
                 const double mr = x.re[I][t], mi = x.im[I][t];
@@ -629,7 +638,7 @@ __device__ __forceinline__ bool inverse4(M4<KB> &x, int n, Lds4<KB> &sh, int lan
         }
 #pragma unroll
         for (int I = 0; I < KB; ++I)
-            if (prow[t] == 4 * I + i && q < kk) x.re[I][t] += 1.0;
+            if (prow[t] == 4 * I + i) x.re[I][t] += 1.0;
     };
     each_of(std::make_integer_sequence<int, KB>(), panel);
 #pragma unroll
@@ -645,7 +654,7 @@ __device__ __forceinline__ bool inverse4(M4<KB> &x, int n, Lds4<KB> &sh, int lan
     return sing;
 }
 
-template <int KB, bool FULL>
+template <int KB>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KB == 1 ? kTinyOcc1 : kTinyOcc)))
 tiny4_kernel(DecimateArgs a) {
     __shared__ Lds4<KB> sh;
@@ -697,11 +706,11 @@ tiny4_kernel(DecimateArgs a) {
                         ey = et.im[I][J];
                     }
                     const int r = 4 * I + i, c = 4 * J + q;
-                    const bool in = FULL || (r < n && c < n);
-                    x.re[I][J] = in ? (r == c ? z.x : 0.0) - ex : 0.0;
+                    const bool in = r < n && c < n;
+                    x.re[I][J] = in ? (r == c ? z.x : 0.0) - ex : r == c ? 1.0 : 0.0;
                     x.im[I][J] = in ? (r == c ? z.y : 0.0) - ey : 0.0;
                 }
-            const bool sing = inverse4<KB, FULL>(x, n, sh, lane);
+            const bool sing = inverse4<KB>(x, n, sh, lane);
             if ((live || f >= 0) && sing) status |= 1;
             if (f >= 0) {
                 // lane 8 b' + r: the terms of orbital r of instance b'
@@ -758,10 +767,7 @@ tiny4_kernel(DecimateArgs a) {
                 for (int J = 0; J < KB; ++J) rsum += cabs_scaled(d.re[I][J], d.im[I][J]);
                 asum += rsum;
             }
-            asum += __shfl_xor(asum, 32, 64);
-            asum += __shfl_xor(asum, 16, 64);
-            asum += __shfl_xor(asum, 2, 64);
-            asum += __shfl_xor(asum, 1, 64);
+            asum = quad_rows_sum(asum);
             const bool conv = asum <= a.accuracy;
             if (live && (conv || it >= a.itermax)) {
                 if (!conv) status |= 2;
@@ -799,23 +805,20 @@ int decimate_tiny_max_n() { return 16; }
 
 int decimate_tiny_run(const DecimateArgs &a, int num_cu, hipStream_t s) {
     if (a.n < 1 || a.n > decimate_tiny_max_n() || num_cu < 1) return -1;
-    // Whole tiles of 4 (FULL) need no masks: 6.6 ms with them, 6.2 ms without
-    // for 80,601 instances of order 16.  Up to one instance a SIMD an instance
+    // Up to one instance a SIMD an instance
     // of order 8 is faster alone in its wave, whose pivots are then uniform
     // (one instance 222 us as one of four, 160 us alone; the same bits, since
     // the steps and the order of every sum are the same).
-    const bool full = a.n % 4 == 0, alone = a.n > 8 || a.ninst <= 4L * num_cu;
+    const bool alone = a.n > 8 || a.ninst <= 4L * num_cu;
     auto one = [&](auto kernel) { return launch_tiny(kernel, a, 1, kTinyOcc, num_cu, s); };
     auto four = [&](auto kernel, int occ) { return launch_tiny(kernel, a, 4, occ, num_cu, s); };
     switch ((a.n + 3) / 4) {
         case 1:
-            if (alone) return full ? one(tiny16_kernel<1, true>) : one(tiny16_kernel<1, false>);
-            return full ? four(tiny4_kernel<1, true>, kTinyOcc1) : four(tiny4_kernel<1, false>, kTinyOcc1);
+            return alone ? one(tiny16_kernel<1>) : four(tiny4_kernel<1>, kTinyOcc1);
         case 2:
-            if (alone) return full ? one(tiny16_kernel<2, true>) : one(tiny16_kernel<2, false>);
-            return full ? four(tiny4_kernel<2, true>, kTinyOcc) : four(tiny4_kernel<2, false>, kTinyOcc);
-        case 3: return full ? one(tiny16_kernel<3, true>) : one(tiny16_kernel<3, false>);
-        default: return full ? one(tiny16_kernel<4, true>) : one(tiny16_kernel<4, false>);
+            return alone ? one(tiny16_kernel<2>) : four(tiny4_kernel<2>, kTinyOcc);
+        case 3: return one(tiny16_kernel<3>);
+        default: return one(tiny16_kernel<4>);
     }
 }
 
