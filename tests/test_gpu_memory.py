@@ -12,6 +12,11 @@ from wannier_tools_amd.surface import SurfaceGF
 
 pytestmark = pytest.mark.gpu
 
+
+@pytest.fixture(autouse=True)
+def automatic_schedule(gpu):
+    gpu.set_schedule("auto")
+
 GIB = 1 << 30
 
 

@@ -527,6 +527,7 @@ def test_mixed_precision_is_fp64_on_the_automatic_schedule(gpu, nw, np_, schedul
     rng = np.random.default_rng(nw)
     kp, om = rng.uniform(-0.5, 0.5, (3, 2)), rng.uniform(-1, 1, 5) * M.EV2HARTREE
     eta = 2e-3 * M.EV2HARTREE
+    gpu.set_schedule("auto")
     want = gpu.spectral_grid(kp, om, eta)
     gpu.set_schedule(schedule)
     try:

@@ -16,6 +16,11 @@ from wannier_tools_amd import model as M
 
 pytestmark = pytest.mark.gpu
 
+
+@pytest.fixture(autouse=True)
+def automatic_schedule(gpu):
+    gpu.set_schedule("auto")
+
 # the last bit of a value, the low and the high word of a double
 STEPS = [2.0 ** -52, 2.0 ** -40, 2.0 ** -19, 2.0 ** -14]
 D, B = 1e-10, 1e300

@@ -11,6 +11,11 @@ from wannier_tools_amd import model as M
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def automatic_schedule(gpu):
+    gpu.set_schedule("auto")
+
+
 def _first_sum(gpu, kp, om, eta):
     """The smallest accuracy with which the first instance takes one iteration."""
     lo, hi = 0, int(np.float64(1e10).view(np.int64))
