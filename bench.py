@@ -543,8 +543,8 @@ def run_c1(args, SurfaceGF) -> dict:
         # the FP64 matrix peak
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": FP64_MFMA_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": achieved / FP64_MFMA_PEAK_TFLOPS, "traffic": None,
-                     "kernel": "decimation stage: small_kernel<16, 1> (one wave per instance, "
-                               "vector ALUs, FP64 peak 78.6 TFLOP/s as the matrix cores')",
+                     "kernel": "decimation stage: tiny16_kernel<4> (one wave per instance, "
+                               "matrix cores and vector ALUs, FP64 peak 78.6 TFLOP/s each)",
                      "flops_per_launch": flops},
     }
     if not args.no_cpu_baseline:
@@ -608,10 +608,10 @@ def run_mixed(args, SurfaceGF) -> dict:
                    "path": "fp64", "members": members},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": FP64_MFMA_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": achieved / FP64_MFMA_PEAK_TFLOPS, "traffic": None,
-                     "kernel": "decimation stages of the four models: small_kernel<8, 1> and "
-                               "small_kernel<32, 8> (Ndim 8, 32; vector ALUs), gj_large_round_kernel<7|14, "
-                               "double> + gemm_large_round_kernel<7|14, double> (Ndim 108 padded to 112, "
-                               "216 padded to 224)",
+                     "kernel": "decimation stages of the four models: tiny4_kernel<2> (Ndim 8), "
+                               "small_kernel (32; vector ALUs), mid_inverse_kernel<14> + mid_gemm_kernel<14> "
+                               "(108 padded to 112), gj_large_round_kernel<14, double> + "
+                               "gemm_large_round_kernel<14, double> (216 padded to 224)",
                      "flops_per_launch": flops},
     }
     if not args.no_cpu_baseline:

@@ -69,7 +69,9 @@ int wtsurf_set_model(wtsurf_ctx *ctx, int nw, int np, int nr, int ijmax,
 int wtsurf_set_stop_rule(wtsurf_ctx *ctx, int itermax, double accuracy);
 
 /* Schedule of the decimation kernels for orders up to 80 (larger orders always
- * run as rounds).  No reference counterpart (the reference solves one
+ * run as rounds).  The rounds' device workspace is kept by the context: up to
+ * 3.1 GB at Ndim 72 and 7.4 GB at Ndim 112, at most a quarter of the free memory
+ * where that is less, and fewer slots where an allocation fails.  No reference counterpart (the reference solves one
  * instance at a time, src/surfstat.f90:123-146).
  *   WTSURF_SCHEDULE_ROUNDS      every iteration is two launches (inverse, GEMMs)
  *                               over a set of instance slots, two sets on two
@@ -78,10 +80,10 @@ int wtsurf_set_stop_rule(wtsurf_ctx *ctx, int itermax, double accuracy);
  *                               workgroup runs whole instances (all iterations,
  *                               final inverses, traces) and takes the next one
  *                               from a device queue.
- *   WTSURF_SCHEDULE_SMALL       Ndim <= 32, FP64: one small workgroup per
- *                               instance on the vector ALUs (no padding to the
- *                               16 x 16 matrix tile), matrices in LDS, several
- *                               workgroups per CU; larger orders and other
+ *   WTSURF_SCHEDULE_SMALL       Ndim <= 32, FP64: whole instances, in the
+ *                               registers of one wave up to Ndim 16 (up to 8
+ *                               four to a wave), beyond that in one workgroup
+ *                               on the vector ALUs; larger orders and other
  *                               precisions run as ROUNDS.
  *   WTSURF_SCHEDULE_AUTO        SMALL where it applies, else ROUNDS. */
 enum {

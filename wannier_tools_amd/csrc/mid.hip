@@ -82,12 +82,13 @@ __device__ __forceinline__ double2 frag_at(const double2 *base, unsigned off) {
 // An FP64 16x16x4 MFMA holds its SIMD for 64 cycles and a complex step is
 // four of them, so one 1 KB operand fragment feeds 256 cycles: the fragments
 // come straight from L2 with no LDS stage, no barrier and no wave waiting for
-// another.  Bound by the matrix cores (busy 74% of the launches' time at
-// order 72, the rest their starts and ends; 287 us for 1024 instances, where
-// the LDS-staged kernel it replaces took 132 us for 256 of them alone).  The
+// another.  Bound by the matrix cores (busy 75% of the launches' time at
+// order 72 alone on the chip, the rest their starts and ends; 576 us for 2048
+// instances, where the LDS-staged kernel it replaces took 132 us for 256).  The
 // fragments are contiguous in memory for the cache's sake: as 64 B pieces of
-// column-major matrices they kept its lookups busy all the time and the same
-// products took 393 us per launch of 1024 for 313.  The MFMAs are issued transposed (the shared matrix as the A
+// column-major matrices they kept its lookups busy all the time, and 1024
+// instances took 393 us where they then took 313 contiguous (288 now).  The
+// MFMAs are issued transposed (the shared matrix as the A
 // operand, the strip as the B operand): the accumulators of the first
 // product, m^T, are then laid out exactly as the B operand of the second, and
 // m1, m2 never leave the registers.
@@ -245,7 +246,8 @@ mid_gemm_kernel(void *work, const MidState *__restrict__ state, int slots, int c
 // eliminates while they update the rest.
 //
 // What it is bound by: an inverse alone is a chain of n pivot searches and
-// reciprocals.  In registers two to three instances fit a CU (in LDS one
+// reciprocals (2048 of order 72 alone on the chip 459 us, its vector ALUs busy 40%
+// of it).  In registers two to three instances fit a CU (in LDS one
 // does), and the updates of the others fill the waits of one's panels.
 template <int KT>
 struct MidGj {
@@ -879,7 +881,9 @@ int dispatch_mid(int kt, const DecimateArgs &a, MidState *in, MidState *out, voi
 
 // Slots per CU and set: a launch ends with its slowest workgroups, so many
 // slots a launch (8192 instances of order 72: 76.6 ms with 512 slots a set,
-// 72.1 with 1024, 69.0 with 2048 and with 4096; one set of 2048: 75.9).
+// 72.1 with 1024, 69.0 with 2048 and with 4096; one set of 2048: 75.9).  The
+// workspace is 0.76 MB a slot at order 72 and 1.8 MB at order 112: 3.1 and 7.4
+// GB for all of them, less where the card has less (decimate_mid_limit).
 constexpr int kMidSlotsPerCu = 8;
 constexpr int kMidRoundsPerBatch = 4;
 
@@ -887,7 +891,7 @@ constexpr int kMidRoundsPerBatch = 4;
 
 // Beyond 112 the inverse's registers (28 complex of a lane at two waves a SIMD)
 // run out.  Between 81 and 112 the kernels with the matrix in global memory that
-// took these orders before: 1500 instances of order 108 59.6 ms, 47.0 here;
+// took these orders before: 1500 instances of order 108 59.6 ms, 47.5 here;
 // 400 of order 96 11.8 and 10.7, of order 81 11.3 and 8.7; one of order 108
 // 9.6 and 4.6.
 int decimate_mid_max_n() { return 112; }

@@ -10,17 +10,17 @@
 //   C(X)  register t: X[4 t + q][i]     the first operand of   X^T r
 // so that R(A B) = mfma(C(B), R(A)) with no movement between lanes: m1 =
 // alpha g and m2 = beta g leave the matrix cores as the operands of m1 alpha,
-// m1 beta, m2 alpha, m2 beta.  R(alpha), R(beta), R(eps_s) and R(eps_t) stay in
-// registers from an instance's set-up to its traces; g, alpha' and beta' are
-// also needed as C and go once through LDS.
+// m1 beta, m2 alpha, m2 beta.  R(eps_s) and R(eps_t) stay in registers from an
+// instance's set-up to its traces; alpha, beta and g lie in LDS, from where they
+// are read as R or as C.
 //
 // Bound by instruction issue: while an FP64 MFMA runs (64 cycles for
 // 16x16x4) its SIMD issues no vector instruction of another wave either
 // (measured: MFMA and FP64, FP32 or integer work of two waves add up), so
 // an iteration at order 16 takes the 7,168 cycles of its 112 MFMA plus about
-// 5,900 of the pivot steps and the rest, 14,000 together.  The kernel it
+// 5,500 of the pivot steps and the rest, 15,000 together.  The kernel it
 // replaces (vector ALUs, one wave per instance, every operand in LDS) was
-// bound by LDS reads: 80,601 instances of order 16 took 10.5 ms, 6.3 ms now;
+// bound by LDS reads: 80,601 instances of order 16 took 10.5 ms, 6.5 ms now;
 // 40,400 of order 8 1.44 ms, 0.80 ms now.  Three waves a SIMD: two with the
 // operands of the products kept in registers took 6.95 ms, three with those
 // registers spilled 9.2.
@@ -807,8 +807,9 @@ int decimate_tiny_run(const DecimateArgs &a, int num_cu, hipStream_t s) {
     if (a.n < 1 || a.n > decimate_tiny_max_n() || num_cu < 1) return -1;
     // Up to one instance a SIMD an instance
     // of order 8 is faster alone in its wave, whose pivots are then uniform
-    // (one instance 222 us as one of four, 160 us alone; the same bits, since
-    // the steps and the order of every sum are the same).
+    // (a call of one instance 222 us as one of four, 160 us alone when the line
+    // was drawn; the same bits, since the steps and the order of every sum are the
+    // same).
     const bool alone = a.n > 8 || a.ninst <= 4L * num_cu;
     auto one = [&](auto kernel) { return launch_tiny(kernel, a, 1, kTinyOcc, num_cu, s); };
     auto four = [&](auto kernel, int occ) { return launch_tiny(kernel, a, 4, occ, num_cu, s); };

@@ -72,8 +72,8 @@ struct PinnedBuf {
 
 // ---------------------------------------------------------------------------
 // Device scratch of wtsurf_surfgreen_1985_noalloc: one instance of order up to
-// kNoallocMaxN (the orders whose Gauss-Jordan matrix sits in LDS), so the call
-// needs no device allocation.  The array lives on every device the library
+// kNoallocMaxN (the orders of the persistent schedule), so the call needs no
+// device allocation.  The array lives on every device the library
 // runs on until the process ends; each device has its own copy at its own
 // address, taken once per device with hipGetSymbolAddress.  Calls on one
 // device share it, so calls that
