@@ -336,6 +336,7 @@ tiny16_kernel(DecimateArgs a) {
             sh.be[c * kLd16 + i] = make_double2(s.x, -s.y);
         }
         et = es;
+        const M16 h0 = es;  // (KS <= 2: H00 stays in registers)
         const int o = a.inst_k ? t : ik + a.nk * (t - ik * a.nomega);
         int it = 1, status = 0;
         // f < 0: the iterations; then G_LL = (z - eps_s)^-1, G_RR = (z -
@@ -348,7 +349,7 @@ tiny16_kernel(DecimateArgs a) {
             M16 x{{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
             for (int v = 0; v < KS; ++v) {
-                const double2 h = H00[i + 16 * (4 * v + q)];
+                const double2 h = KS <= 2 ? make_double2(h0.re[v], h0.im[v]) : H00[i + 16 * (4 * v + q)];
                 double ex = (es.re[v] + et.re[v]) - h.x, ey = (es.im[v] + et.im[v]) - h.y;
                 if (f == 0) {
                     ex = es.re[v];
