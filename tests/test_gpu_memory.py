@@ -83,8 +83,8 @@ def test_qpi_sums_give_large_buffers_back(gpu):
 
 
 def test_hamiltonians_with_little_memory_left(gpu, fill):
-    """A list of k points whose H00 and H01 fit the card but not a whole piece of
-    the download beside them: bit for bit as with memory to spare."""
+    """A list of k points whose H00 and H01 fit the card with little beside them:
+    bit for bit as with memory to spare."""
     n, nk = 96, 500
     irvec, hr = M.synthetic_model(n, 1, 0.4, M.decay_l2(1.5), seed=96).surface_cell()
     k = np.random.default_rng(4).uniform(-0.5, 0.5, (nk, 2))
@@ -93,7 +93,7 @@ def test_hamiltonians_with_little_memory_left(gpu, fill):
     ctx = SurfaceGF(0)
     try:
         ctx.set_model_arrays(n, 1, irvec, hr)
-        fill(200 << 20)  # 147 MB of H00 and H01, 2 x 64 MiB a piece
+        fill(200 << 20)  # 147 MB of H00 and H01
         print("little memory", free_memory(), flush=True)
         got = ctx.ham_qlayer2qlayer(k)
     finally:

@@ -83,7 +83,7 @@ def test_kpath_jdos_at_path_edges(gpu, nk):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,nk", [(3, 70), (16, 5), (200, 110)])
 def test_ham_of_many_k_points(gpu, n, nk):
-    """A whole list of k points (at n = 200 more than one piece of 64 MiB)
+    """A whole list of k points (at n = 200 one pair to a piece of the download)
     against the points one by one, bit for bit."""
     print("ham", n, nk, flush=True)
     irvec, hr = M.synthetic_model(n, 1, 0.4, M.decay_l2(1.5), seed=n).surface_cell()

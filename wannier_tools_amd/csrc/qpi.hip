@@ -21,10 +21,10 @@
 // R2 rows of a_f over the row of E_f, one LDS read of a row and one of E
 // (broadcast) for 8 R2 multiply-adds, where a thread per (p1, p2) took two
 // reads for each: at 257 x 257, moduli 256 and four fields, 6.97 ms, bound by
-// the LDS reads, and 0.74 ms now
-// (rows staged one load at a time a thread 0.79, windows of two rows 0.81).  Rows go in groups of G values of c2, one per group of
-// threads; the sum over c2 is cut into slices so that there are workgroups for
-// the whole chip, and expand_kernel adds the slices in order.  Bound by the
+// the LDS reads, and 0.73 ms now (rows staged one load at a time a thread 0.79,
+// windows of two rows 0.81).  Rows go in groups of G values of c2, one per group
+// of threads; the sum over c2 is cut into slices so that there are workgroups
+// for the whole chip, and expand_kernel adds the slices in order.  Bound by the
 // FP64 vector ALUs.
 //
 // 2. Linear autocorrelation along a k path, per energy (surfstat_jdos,

@@ -143,19 +143,19 @@ __device__ __forceinline__ M16 read_c16(const double2 *m, int i, int q) {
 }
 
 // x = R(X), the identity (KS <= 2: zero) from row and column n to 4 KS: X^-1 to
-// sh.g in natural order, the identity from there on (the identity of order n if a pivot column is zero or NaN;
-// returns true then).  Gauss-Jordan with
-// partial pivoting on |re| + |im| over the rows not yet used (the izamax rule
-// of zgesv, the lowest row on ties), rows never swapped: step c's pivot row p keeps its values unscaled, standing for
-// 1/pivot times itself, takes every later step like any other row and is
-// scaled once at the end; element (row r, column c) is then X^-1[step of
-// r][pivot row of step c].  Rows and columns from n on hold the identity, whose
-// steps change nothing, or (KS <= 2: the time of one instance, and what the
-// registers of larger orders do not allow) zero, whose steps are left out.
-// Columns are eliminated in panels of 4, one register of
-// every lane, and the panel is applied to the rest as X += M T by four MFMA,
-// M the panel's columns (with the distance from 1 where a pivot row meets
-// its own column) and T its pivot rows.
+// sh.g in natural order, the identity from there on (the identity of order n if
+// a pivot column is zero or NaN; returns true then).  Gauss-Jordan with partial
+// pivoting on |re| + |im| over the rows not yet used (the izamax rule of zgesv,
+// the lowest row on ties), rows never swapped: step c's pivot row p keeps its
+// values unscaled, standing for 1/pivot times itself, takes every later step
+// like any other row and is scaled once at the end; element (row r, column c) is
+// then X^-1[step of r][pivot row of step c].  Rows and columns from n on hold the
+// identity, whose steps change nothing, or (KS <= 2: the time of one instance,
+// and what the registers of larger orders do not allow) zero, whose steps are
+// left out.  Columns are eliminated in panels of 4, one register of every lane,
+// and the panel is applied to the rest as X += M T by four MFMA, M the panel's
+// columns (with the distance from 1 where a pivot row meets its own column) and T
+// its pivot rows.
 template <int KS>
 __device__ __forceinline__ bool inverse16(M16 &x, int n, Lds16 &sh, int lane) {
     const int i = lane & 15, q = lane >> 4;
